@@ -902,7 +902,7 @@ int potg_direct_sum(potg_ctx* c, uint32_t inst, const uint32_t* idx, size_t n, d
             vs[k] = inv[off + idx[s0 + k]];
         }
         HIPCHK(hipMemcpyAsync(b.q_self, vs.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
-        launch_direct_sum(b, inst, m, c->stream);
+        launch_direct_sum(b, inst, (uint32_t)c->cfg[inst].N, m, c->stream);
         HIPCHK(hipMemcpyAsync(E + 3 * s0, b.q_out, 3 * sizeof(double) * m, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
     }
