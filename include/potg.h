@@ -151,14 +151,17 @@ typedef struct potg_stats_t {
    64-target tiles per CU (half the particles are targets): the float32
    walk sweeps whole ranges with 64 targets per wavefront on 8 blocks per CU
    from 16 tiles per CU (about 0.5M particles), on 2 blocks per CU from 1
-   tile per CU, and below that takes 8 targets per wavefront on 2 blocks
-   per CU; the float64 walk takes 64 targets on 8 blocks per CU from 16
+   tile per CU, and below that takes 8 targets per wavefront, one after the
+   other; the float64 walk takes 64 targets on 8 blocks per CU from 16
    tiles per CU, 4 below. */
 typedef struct potg_tuning {
-    uint32_t walk_blocks; /* blocks (4 wavefronts each) of the persistent walk */
+    uint32_t walk_blocks; /* blocks (4 wavefronts each) of the persistent walk;
+                             not used by a walk of 8 targets per wavefront */
     uint32_t group;       /* float32 walk: targets per wavefront, 8, 16 or 64;
-                             with 8 or 16 the wavefront evaluates 8 or 4
-                             children per target at once */
+                             with 8 (at most: fewer in a small context) they are
+                             walked one after the other, 64 nodes at once; with
+                             16 the wavefront evaluates 4 children per target
+                             at once */
     uint32_t variant;     /* float32 walk with 64 targets: 0 visits a range's
                              cells until some lanes open one, 1 sweeps every
                              range whole before descending */
@@ -235,7 +238,7 @@ int potg_phi_at(potg_ctx* ctx, uint32_t inst, const double* xyz, size_t n, doubl
    capture, tight serving loops, harnesses that forbid hipMalloc.  No
    counterpart in the reference.  d_xyz (3 n doubles) and d_phi (n doubles)
    are device memory; the call allocates nothing (its scratch is a fixed
-   array of about 0.5 MB per device, held until the process ends), does not
+   array of 0.5 MB per device, held until the process ends), does not
    synchronise and enqueues on `stream` (a hipStream_t; NULL for the
    context's stream).  n may be at most POTG_NOALLOC_MAX_POINTS, else
    POTG_ERR_ARG.  Calls that overlap on one GPU share the scratch and race.

@@ -316,11 +316,6 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
             } else {
                 io.out[k] = ph;
             }
-            if (COUNT && io.counts) {
-                io.counts[3 * k] = ncell;
-                io.counts[3 * k + 1] = nleaf;
-                io.counts[3 * k + 2] = nopen;
-            }
         }
         tot_cell += ncell;
         tot_leaf += nleaf;
@@ -897,6 +892,326 @@ __global__ __launch_bounds__(BT) void k_walk32s(const InstParams* __restrict__ P
     }
 }
 
+// ---- one target per wavefront ---------------------------------------------
+//
+// The 64 lanes of a wavefront test 64 nodes against one target: up to 8
+// child ranges are taken off an LDS stack at once, lane = 8 range + child,
+// and the ranges of the children that the target opens are pushed back.
+// The interaction set is the reference's, and no lane works for another
+// target's: a wavefront that walks for several targets steps through the
+// union of their sets, which for 64 neighbours is 2.3 (theta 0.5, 2M
+// particles) to 4 times one target's, and for scattered points many times it.
+// The loads are 32- or 48-byte gathers from L2, 8 contiguous records a range.
+// Step walk, mixed, theta 0.5: 16k particles 0.36 (8 targets against 8
+// children at once) -> 0.028 ms.  The force at 65536 scattered points of 1M
+// particles with its tree build 12.6 -> 3.4 ms, the potential at 2200 grid
+// points of 150k particles 2.37 -> 0.08 ms (64 points shared a traversal).
+//
+// Targets of a wavefront (per_wave at most 8) are read together, lane by
+// lane, and walked one after the other.  Neighbouring blocks, which the
+// hardware deals to the 8 XCDs in turn, take targets from 8 separate
+// stretches of the list, so that each XCD's L2 holds one region's nodes.
+//
+// float32: each lane sums its own interactions, flushed every 4 passes into a
+// compensated sum; the lanes' sums are added in float64, in a fixed order.
+// float64: plain float64 sums; 1 / r from the hardware's reciprocal square
+// root, refined.  Every result depends on its target and the tree alone.
+constexpr uint32_t XCDS = 8;
+constexpr int NS1 = 632;
+// below this the stack takes 8 ranges at a time (which leaves at most 56
+// more), above it one, depth first, which adds at most 7 a level
+constexpr int SP1_WIDE = NS1 - 7 * MAXD - 56;
+
+// 1 / sqrt(r2) to the last bits: the hardware's value (relative error below
+// 2^-23), then (1 - e)^(-1/2) = 1 + e/2 + 3/8 e^2 + O(e^3), e = 1 - r2 r^2
+__device__ inline double rsqrt64(double r2)
+{
+    const double r = __builtin_amdgcn_rsq(r2);
+    const double e = __builtin_fma(-r2 * r, r, 1.0);
+    return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
+}
+
+// row_shr 1, 2, 4, 8 added up: lane 15 of each 16-lane row holds its sum
+template <int CTRL>
+__device__ inline double dpp_add(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+    return v + __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+__device__ inline double row_sum(double v)
+{
+    return dpp_add<0x118>(dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(v))));
+}
+// a's lanes 32-63 change places with b's 0-31 (or a's odd rows with b's
+// even ones); the sum of the two
+template <bool HALF>
+__device__ inline double swap_add(double a, double b)
+{
+    const uint64_t ua = (uint64_t)__double_as_longlong(a), ub = (uint64_t)__double_as_longlong(b);
+    const uint32_t al = (uint32_t)ua, ah = (uint32_t)(ua >> 32), bl = (uint32_t)ub,
+                   bh = (uint32_t)(ub >> 32);
+    const auto lo = HALF ? __builtin_amdgcn_permlane32_swap(al, bl, false, false)
+                         : __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto hi = HALF ? __builtin_amdgcn_permlane32_swap(ah, bh, false, false)
+                         : __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    return __longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1]));
+}
+// three sums over the wavefront at once: x in lane 15, z in lane 31, y in
+// lane 47
+__device__ inline double wave_sum3(double x, double y, double z)
+{
+    return row_sum(swap_add<false>(swap_add<true>(x, y), swap_add<true>(z, 0.0)));
+}
+__device__ inline uint32_t wave_sum_u(uint32_t v)
+{
+    for (int d = 1; d < WAVE; d <<= 1) v += __shfl_xor(v, d, WAVE);
+    return v;
+}
+__device__ inline bool lane_of(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+template <bool F64>
+struct Walk1Rec { using type = NodeRec32; };
+template <>
+struct Walk1Rec<true> { using type = NodeRec64; };
+
+template <bool F64, int MODE, int KIND, bool DIP, bool COUNT>
+__global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, Globals* g,
+                                              PState st,
+                                              const typename Walk1Rec<F64>::type* __restrict__ rec,
+                                              WalkIO io, uint32_t per_wave)
+{
+    using Rec = typename Walk1Rec<F64>::type;
+    // float32: a range's first record counted in 16-byte units (2 n_rec stays
+    // below 2^32 for any context that fits the device), an address of one add
+    constexpr uint32_t U = F64 ? 1 : 2;
+    // a range's first record (times U) and its count; below the stack 8
+    // entries without children, so that a pass always reads 8
+    __shared__ uint2 s_mem[NW][8 + NS1];
+    const int wv = threadIdx.x / WAVE;
+    uint2* const s_stk = &s_mem[wv][8];
+    const uint32_t lane = __lane_id();
+    const uint32_t ci = lane & 7u;
+    const uint2* const s_top = s_stk - 1 - (lane >> 3);  // the lane's range at sp = 0
+    const uint32_t ntg = (MODE == MODE_STEP) ? *io.n_targets_dev : io.n_pts;
+    if (rfl(step_failed(g) ? 1u : 0u)) return;
+    if (lane < 8u) s_mem[wv][lane] = make_uint2(0u, 0u);
+    unsigned long long tot_cell = 0, tot_leaf = 0, tot_open = 0, tot_pops = 0;
+    const uint32_t nblk = (ntg + NW * per_wave - 1) / (NW * per_wave);
+    const uint32_t per_xcd = (nblk + XCDS - 1) / XCDS;
+
+    for (uint32_t b = blockIdx.x; b / XCDS < per_xcd; b += gridDim.x) {
+        const uint32_t tile = (b % XCDS) * per_xcd + b / XCDS;
+        if (tile >= nblk) continue;
+        // the wavefront's targets, one a lane
+        const uint32_t k0 = (tile * NW + wv) * per_wave;
+        uint32_t l_inst, l_self;
+        double l_x, l_y, l_z;
+        const bool valid = load_target<MODE>(P, st, io, k0 + lane, lane < per_wave ? ntg : 0u, l_inst,
+                                             l_self, l_x, l_y, l_z);
+        float l_fx = 0.f, l_fy = 0.f, l_fz = 0.f, l_soft2 = 0.f;
+        if constexpr (!F64) {
+            const InstParams& p = P[l_inst];
+            l_fx = (float)((l_x - p.R) * p.invR);
+            l_fy = (float)((l_y - p.R) * p.invR);
+            l_fz = (float)((l_z - p.R) * p.invR);
+            l_soft2 = (float)(p.soft2 * p.invR * p.invR);
+        }
+        for (uint64_t todo = ballot(valid); todo; todo &= todo - 1u) {
+            const uint32_t src = (uint32_t)__builtin_ctzll(todo);
+            const uint32_t k = k0 + src;
+            const uint32_t gi = bcast_u(l_inst, src), self = bcast_u(l_self, src);
+            const InstParams& p = P[gi];
+            const bool dip = DIP && p.dipoles && (F64 ? (const void*)io.dip64 : (const void*)io.dip32);
+            float tx = 0.f, ty = 0.f, tz = 0.f, soft2f = 0.f;
+            double dtx = 0.0, dty = 0.0, dtz = 0.0, theta2 = 0.0, soft2 = 0.0;
+            if constexpr (F64) {
+                dtx = bcast_d(l_x, src);
+                dty = bcast_d(l_y, src);
+                dtz = bcast_d(l_z, src);
+                theta2 = p.theta2;
+                soft2 = p.soft2;
+            } else {
+                tx = bcast_f(l_fx, src);
+                ty = bcast_f(l_fy, src);
+                tz = bcast_f(l_fz, src);
+                soft2f = bcast_f(l_soft2, src);
+            }
+            double ex = 0.0, ey = 0.0, ez = 0.0;  // float64: the sums (ex: a potential's)
+            float fx = 0.f, fy = 0.f, fz = 0.f, kx = 0.f, ky = 0.f, kz = 0.f;
+            uint32_t ncell = 0, nleaf = 0, nopen = 0, loads = 0;
+            // the root alone; an empty instance has no nodes
+            if (lane == 0) s_stk[0] = make_uint2(gi * U, 1u);
+            __builtin_amdgcn_wave_barrier();
+            int sp = rfl(p.tree_n) != 0u ? 1 : 0;
+            while (sp > 0) {
+                float px = 0.f, py = 0.f, pz = 0.f;
+                for (int u = 0; u < 4 && sp > 0; u++) {
+                    const bool wide = sp <= SP1_WIDE;
+                    int take = wide ? (sp < 8 ? sp : 8) : 1;
+                    asm("" : "+s"(take));
+                    // the lanes past a range, below the stack or past `take`
+                    // read a record that is there and add nothing; lane sets
+                    // are scalar masks
+                    const uint2 en = s_top[sp];
+                    const uint64_t m_in = ballot(ci < en.y) & (wide ? ~0ull : 0xffull);
+                    const uint32_t w = en.x + (lane_of(m_in) ? ci * U : 0u);
+                    const int base = sp - take;
+                    loads += (uint32_t)take;
+                    const uint32_t wr = w / U;
+                    Rec r;
+                    if constexpr (F64) r = rec[w];
+                    else r = *(const Rec*)((const uint4*)rec + w);
+                    const uint64_t m_leaf = ballot(r.cnt == LEAF);
+                    const uint64_t m_own = KIND == KIND_PHI ? 0ull : m_leaf & ballot(r.part == self);
+                    uint64_t m_use, m_open;
+                    if constexpr (F64) {
+                        const double dx = dtx - r.cx, dy = dty - r.cy, dz = dtz - r.cz;
+                        // the reference's opening test, in its operations
+                        const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
+                        const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
+                        m_use = m_in & (m_acc | m_leaf) & ~m_own;
+                        if (KIND == KIND_FIELD) {
+                            const uint64_t m_hit = m_use & m_leaf & ballot(d2 == 0.0);
+                            if (m_hit) {
+                                if (lane_of(m_hit)) raise_err(g, KERR_COINCIDENT, self);
+                                m_use &= ~m_hit;
+                            }
+                        }
+                        m_open = m_in & ~(m_acc | m_leaf);
+                        const bool use = lane_of(m_use);
+                        const double r2 = lane_of(m_leaf) ? d2 + soft2 : d2;
+                        double inv = rsqrt64(r2);
+                        if (KIND != KIND_FIELD && r2 == 0.0) inv = __builtin_inf();
+                        inv = use ? inv : 0.0;
+                        const double q = (double)r.q;
+                        if (KIND == KIND_FIELD) {
+                            const double inv2 = inv * inv, inv3 = inv2 * inv;
+                            if (DIP && dip) {
+                                // zero for a leaf
+                                const double* dp = io.dip64 + 3 * (size_t)wr;
+                                const double pdx = dp[0], pdy = dp[1], pdz = dp[2];
+                                const double rpd2 =
+                                    __builtin_fma(dx, pdx, __builtin_fma(dy, pdy, dz * pdz)) * inv2;
+                                const double ca = __builtin_fma(3.0, rpd2, q);
+                                ex = __builtin_fma(inv3, __builtin_fma(ca, dx, -pdx), ex);
+                                ey = __builtin_fma(inv3, __builtin_fma(ca, dy, -pdy), ey);
+                                ez = __builtin_fma(inv3, __builtin_fma(ca, dz, -pdz), ez);
+                            } else {
+                                const double ca = q * inv3;
+                                ex = __builtin_fma(ca, dx, ex);
+                                ey = __builtin_fma(ca, dy, ey);
+                                ez = __builtin_fma(ca, dz, ez);
+                            }
+                        } else {
+                            double ph = q * inv;
+                            if (DIP && dip) {
+                                // zero for a leaf
+                                const double* dp = io.dip64 + 3 * (size_t)wr;
+                                const double rdp =
+                                    __builtin_fma(dx, dp[0], __builtin_fma(dy, dp[1], dz * dp[2]));
+                                if (!lane_of(m_leaf)) ph = __builtin_fma(rdp * inv, inv * inv, ph);
+                            }
+                            ex += use ? ph : 0.0;
+                        }
+                    } else {
+                        const float dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
+                        const float d2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+                        // a leaf's size2 is zero: a leaf at float32 distance
+                        // zero adds nothing
+                        const uint64_t m_acc = ballot(!(d2 <= r.size2));
+                        m_use = m_in & m_acc & ~m_own;
+                        m_open = m_in & ~(m_acc | m_leaf);
+                        const float r2 = d2 + (lane_of(m_leaf) ? soft2f : 0.f);
+                        const float inv = lane_of(m_use) ? __builtin_amdgcn_rsqf(r2) : 0.f;
+                        const float inv2 = inv * inv, inv3 = inv2 * inv;
+                        if (DIP && dip) {
+                            const float4 pd = io.dip32[wr];
+                            const float rpd2 =
+                                __builtin_fmaf(dx, pd.x, __builtin_fmaf(dy, pd.y, dz * pd.z)) * inv2;
+                            const float ca = __builtin_fmaf(3.f, rpd2, r.q);
+                            px = __builtin_fmaf(inv3, __builtin_fmaf(ca, dx, -pd.x), px);
+                            py = __builtin_fmaf(inv3, __builtin_fmaf(ca, dy, -pd.y), py);
+                            pz = __builtin_fmaf(inv3, __builtin_fmaf(ca, dz, -pd.z), pz);
+                        } else {
+                            const float ca = r.q * inv3;
+                            px = __builtin_fmaf(ca, dx, px);
+                            py = __builtin_fmaf(ca, dy, py);
+                            pz = __builtin_fmaf(ca, dz, pz);
+                        }
+                    }
+                    if (COUNT) {
+                        const uint64_t m_chg = ballot(dip ? r.part != 0u : r.q != 0);
+                        ncell += lane_of(m_use & ~m_leaf & m_chg) ? 1u : 0u;
+                        nleaf += lane_of(m_use & m_leaf) ? 1u : 0u;
+                        nopen += lane_of(m_open) ? 1u : 0u;
+                    }
+                    // push the opened ranges
+                    const uint64_t m_bad = m_open & ballot(r.first + r.cnt > io.n_rec);
+                    const int ns = __popcll(m_open);
+                    if (m_bad || base + ns > NS1 || loads > io.n_rec) {
+                        if (lane_of(m_bad)) raise_err(g, KERR_CAPACITY, wr);
+                        if (!m_bad && lane == 0) raise_err(g, KERR_DEPTH, gi);
+                        sp = 0;
+                    } else {
+                        const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(m_open >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m_open, 0u));
+                        if (lane_of(m_open)) s_stk[base + (int)below] = make_uint2(r.first * U, r.cnt);
+                        sp = base + ns;
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                }
+                if constexpr (!F64) {
+                    kahan_add(fx, kx, px);
+                    kahan_add(fy, ky, py);
+                    kahan_add(fz, kz, pz);
+                }
+            }
+            if constexpr (!F64) {
+                ex = (double)fx - (double)kx;
+                ey = (double)fy - (double)ky;
+                ez = (double)fz - (double)kz;
+            }
+            const double K = F64 ? QE / K4PE0 : QE / (K4PE0 * p.R * p.R);
+            const double e = KIND == KIND_FIELD ? wave_sum3(ex, ey, ez) : wave_sum3(ex, 0.0, 0.0);
+            // x from lane 15, z from 31, y from 47; a potential from lane 15
+            if ((lane & 15u) == 15u && lane < (KIND == KIND_FIELD ? 48u : 16u)) {
+                double* o = io.out + (KIND == KIND_FIELD
+                                          ? 3 * (size_t)k + (lane == 15u ? 0u : (lane == 31u ? 2u : 1u))
+                                          : (size_t)k);
+                *o = (io.acc ? *o : 0.0) + K * e;
+            }
+            if (COUNT && io.counts) {
+                const uint32_t nc = wave_sum_u(ncell), nl = wave_sum_u(nleaf), no = wave_sum_u(nopen);
+                if (lane == 0) {
+                    io.counts[3 * k] = nc;
+                    io.counts[3 * k + 1] = nl;
+                    io.counts[3 * k + 2] = no;
+                }
+            }
+            tot_cell += ncell;
+            tot_leaf += nleaf;
+            tot_open += nopen;
+            tot_pops += loads;
+        }
+    }
+    if (COUNT && KIND == KIND_FIELD) {
+        for (int d = 1; d < WAVE; d <<= 1) {
+            tot_cell += __shfl_xor(tot_cell, d, WAVE);
+            tot_leaf += __shfl_xor(tot_leaf, d, WAVE);
+            tot_open += __shfl_xor(tot_open, d, WAVE);
+        }
+        if (lane == 0) {
+            atomicAdd(&g->n_cell, tot_cell);
+            atomicAdd(&g->n_leaf, tot_leaf);
+            atomicAdd(&g->n_open, tot_open);
+            atomicAdd(&g->n_pops, tot_pops);
+        }
+    }
+}
+
 // ---- grouped float32 walk ----------------------------------------------
 //
 // A wavefront serves a group of K targets (consecutive in key order, so
@@ -919,7 +1234,7 @@ __global__ __launch_bounds__(BT) void k_walkg(const InstParams* __restrict__ P, 
                                                PState st, const NodeRec32* __restrict__ rec,
                                                WalkIO io)
 {
-    static_assert(K == 8 || K == 16, "group width");
+    static_assert(K == 16, "group width");
     constexpr uint32_t S = WAVE / K;
     constexpr uint32_t KMASK = (1u << K) - 1u;
     // a visit pops one range and pushes at most 8, so the stack holds at
@@ -1402,9 +1717,37 @@ void launch_walk_init(Bufs& b, hipStream_t s)
     k_grain_init<MODE_STEP, KIND_FIELD><<<(nt + BT - 1) / BT, BT, 0, s>>>(b.P, b.S, b.st, io);
 }
 
+// n: targets at most (step walks: half of it in most steps).  Targets per
+// wavefront: as many, up to 8, as still leave four rounds of 8 blocks per CU
+// -- a target alone keeps every wavefront of a small context busy, several
+// share the latency of reading the targets.  Walk ms at 1 / 2 / 4 / 8: 16k
+// particles 0.028 / 0.029 / 0.042 / 0.071, 150k (theta 0.8) 0.103 / 0.089 /
+// 0.088 / 0.094, 2M 2.70 / 2.57 / 2.51 / 2.47.
+template <bool F64, int MODE, int KIND, bool COUNT>
+static void launch_walk1(Bufs& b, uint32_t n, const WalkIO& io, hipStream_t s)
+{
+    const uint32_t round = NW * 8u * (uint32_t)device_cus();
+    uint32_t pw = (MODE == MODE_STEP ? n / 2 : n) / (4u * round);
+    pw = pw < 1 ? 1 : (pw > 8 ? 8 : pw);
+    uint32_t blocks = (n + NW * pw - 1) / (NW * pw);
+    blocks = (blocks + XCDS - 1) / XCDS * XCDS;
+    if (blocks > 65536u) blocks = 65536u;
+#define POTG_W1(DIP, REC) \
+    k_walk1<F64, MODE, KIND, DIP, COUNT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, REC, io, pw)
+    if constexpr (F64) {
+        if (b.dip64) POTG_W1(true, b.rec64);
+        else POTG_W1(false, b.rec64);
+    } else {
+        if (b.dip32) POTG_W1(true, b.rec32);
+        else POTG_W1(false, b.rec32);
+    }
+#undef POTG_W1
+}
+
 // float32 field walk of the chosen shape: the group criterion
-// (k_walk32grp), groups of 8 or 16 targets (k_walkg), or 64 targets stepping
-// through the children (k_walk32); instantiated with dipole support only
+// (k_walk32grp), one target per wavefront at a time (k_walk1: group 8, and
+// point queries unless another shape was set), groups of 16 targets
+// (k_walkg), or 64 targets stepping through the children (k_walk32s, k_walk32); instantiated with dipole support only
 // for contexts holding DIPOLES instances, and with interaction counting
 // (COUNT) for point queries and for step walks while the context counts
 template <int MODE, bool COUNT>
@@ -1415,12 +1758,14 @@ static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
     if (b.precision == POTG_MIXED_GROUP) {
         if (dip) POTG_W32((k_walk32grp<MODE, true, COUNT>));
         else POTG_W32((k_walk32grp<MODE, false, COUNT>));
+    } else if (b.group == 8 || (MODE == MODE_POINTS && b.group == 64 && b.variant == 1)) {
+        // points come in the caller's order, as often as not scattered
+        launch_walk1<false, MODE, KIND_FIELD, COUNT>(b, MODE == MODE_STEP ? b.t_cap : io.n_pts, io, s);
     } else if (b.group == 64 && b.variant == 1) {
-        if (dip) POTG_W32((k_walk32s<MODE, true, COUNT>));
-        else POTG_W32((k_walk32s<MODE, false, COUNT>));
-    } else if (b.group == 8) {
-        if (dip) POTG_W32((k_walkg<8, MODE, true, COUNT>));
-        else POTG_W32((k_walkg<8, MODE, false, COUNT>));
+        if constexpr (MODE == MODE_STEP) {
+            if (dip) POTG_W32((k_walk32s<MODE, true, COUNT>));
+            else POTG_W32((k_walk32s<MODE, false, COUNT>));
+        }
     } else if (b.group == 16) {
         if (dip) POTG_W32((k_walkg<16, MODE, true, COUNT>));
         else POTG_W32((k_walkg<16, MODE, false, COUNT>));
@@ -1450,7 +1795,7 @@ static void launch_walk64c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
 template <int MODE, int KIND>
 static void launch_walk64(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
 {
-    if (MODE == MODE_POINTS || b.count) launch_walk64c<MODE, KIND, true>(b, blocks, io, s);
+    if (b.count) launch_walk64c<MODE, KIND, true>(b, blocks, io, s);
     else launch_walk64c<MODE, KIND, false>(b, blocks, io, s);
 }
 
@@ -1471,24 +1816,25 @@ void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s)
     io.pt_self = b.q_self;
     io.n_pts = n;
     io.out = b.q_out;
-    io.acc = 1;
+    io.acc = b.any_spheroid;
     io.counts = kind == 0 ? b.q_counts : nullptr;
     io.tile_ctr = &b.g->tile_ctr2;
     io.n_rec = b.n_rec;
     io.dip64 = b.dip64;
     io.dip32 = b.dip32;
-    k_reset_tiles<<<1, 1, 0, s>>>(&b.g->tile_ctr2);
     const uint32_t nb = (n + BT - 1) / BT ? (n + BT - 1) / BT : 1;
-    const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
     if (kind == 1) {
-        k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-        launch_walk64<MODE_POINTS, KIND_PHI>(b, blocks, io, s);
+        if (io.acc) k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
+        launch_walk1<true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
+        return;
+    }
+    if (io.acc) k_grain_init<MODE_POINTS, KIND_FIELD><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
+    if (b.precision) {
+        k_reset_tiles<<<1, 1, 0, s>>>(&b.g->tile_ctr2);
+        const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
+        launch_walk32<MODE_POINTS>(b, blocks, io, s);
     } else {
-        k_grain_init<MODE_POINTS, KIND_FIELD><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-        if (b.precision)
-            launch_walk32<MODE_POINTS>(b, blocks, io, s);
-        else
-            launch_walk64<MODE_POINTS, KIND_FIELD>(b, blocks, io, s);
+        launch_walk1<true, MODE_POINTS, KIND_FIELD, true>(b, n, io, s);
     }
 }
 
@@ -1605,15 +1951,13 @@ void launch_chi_b(Bufs& b, hipStream_t s)
 // ---- point potentials with no allocation (potg_phi_at_noalloc) -----------
 //
 // The walk of a point query reads, besides the caller's points and result
-// array, a tile counter and an instance and excluded-slot entry per point.
-// For callers that cannot allocate, that scratch is this array: word 0 is
-// the tile counter, then NOALLOC_MAX points' instances, then their excluded
-// slots (all NONE: a potential counts every leaf).  Each device holds one
+// array, an instance and excluded-slot entry per point.  For callers that
+// cannot allocate, that scratch is this array: the points' instances, then
+// their excluded slots (all NONE: a potential counts every leaf).  Each device holds one
 // copy until the process ends; the host reaches it only through the address
 // hipGetSymbolAddress gives on that device.  Calls that overlap on one device
 // share it and race.
-constexpr uint32_t NOALLOC_HEAD = 64;  // words before the per-point arrays
-constexpr uint32_t NOALLOC_WORDS = NOALLOC_HEAD + 2 * POTG_NOALLOC_MAX_POINTS;
+constexpr uint32_t NOALLOC_WORDS = 2 * POTG_NOALLOC_MAX_POINTS;
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
 
 namespace {
@@ -1621,10 +1965,9 @@ namespace {
 __global__ void k_noalloc_prep(uint32_t* __restrict__ scr, uint32_t inst, uint32_t n)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k == 0) scr[0] = 0u;  // the walk's tile counter starts from zero
     if (k < n) {
-        scr[NOALLOC_HEAD + k] = inst;
-        scr[NOALLOC_HEAD + POTG_NOALLOC_MAX_POINTS + k] = NONE;
+        scr[k] = inst;
+        scr[POTG_NOALLOC_MAX_POINTS + k] = NONE;
     }
 }
 
@@ -1653,19 +1996,17 @@ void launch_phi_noalloc(Bufs& b, uint32_t* scr, uint32_t inst, const double* pts
 {
     WalkIO io{};
     io.pts = pts;
-    io.pt_inst = scr + NOALLOC_HEAD;
-    io.pt_self = scr + NOALLOC_HEAD + POTG_NOALLOC_MAX_POINTS;
+    io.pt_inst = scr;
+    io.pt_self = scr + POTG_NOALLOC_MAX_POINTS;
     io.n_pts = n;
     io.out = out;
-    io.acc = 1;
-    io.tile_ctr = scr;
+    io.acc = b.any_spheroid;
     io.n_rec = b.n_rec;
     io.dip64 = b.dip64;
     const uint32_t nb = (n + BT - 1) / BT ? (n + BT - 1) / BT : 1;
-    const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
     k_noalloc_prep<<<nb, BT, 0, s>>>(scr, inst, n);
-    k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-    launch_walk64<MODE_POINTS, KIND_PHI>(b, blocks, io, s);
+    if (io.acc) k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
+    launch_walk1<true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
 }
 
 }  // namespace potg
