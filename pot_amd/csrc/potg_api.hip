@@ -190,6 +190,22 @@ void fill_params(InstParams& p, const potg_config& k)
     for (int s = 0; s < 3; s++) p.first_idx[s] = NONE;
 }
 
+// Whether the float64 walk gives each target a wavefront of its own (k_walk1)
+// or 64 to one (k_walk64).  Alone, no lane works for another's target, but
+// every node comes through the L1 once per target; 64 neighbours share the
+// loads, and the more of their nodes the smaller theta, but 64-target tiles
+// are too few to fill a device below a few hundred thousand particles.
+// Step walk, ms, alone / together: 150k particles theta 0.8 0.10 / 0.62, theta
+// 0.14 DIPOLES 5.7 / 15.5; 500k theta 0.3 3.8 / 5.6, 0.2 11.9 / 13.1, 0.14
+// 33.9 / 26.2 (all DIPOLES); 2M theta 0.5 2.9 / 4.6, 0.3 10.9 / 12.0, 0.14
+// DIPOLES 204 / 77.  By an instance's own values, so that its walk is the same
+// alone and in a batch.
+int lone64_rule(const InstParams& p)
+{
+    const double theta = sqrt(p.theta2);
+    return theta >= 0.25 || (theta >= 0.17 && p.tree_n < 800000u) || p.tree_n < 250000u;
+}
+
 // chi_b sampling point of the one worker (measure_chi_b, pot.c:2257-2275)
 void chi_point(InstParams& p)
 {
@@ -387,6 +403,8 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
         c->hp[i].offset = off;
         c->hp[i].tree_begin = tb;
         c->hp[i].tree_n = (uint32_t)configs[i].N - (configs[i].geometry != POTG_SPHERE ? 1 : 0);
+        c->hp[i].lone64 = lone64_rule(c->hp[i]);
+        b.n_lone64 += c->hp[i].lone64 != 0;
         off += (uint32_t)configs[i].N;
         tb += c->hp[i].tree_n;
     }

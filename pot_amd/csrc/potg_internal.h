@@ -21,6 +21,7 @@ struct Bufs {
     uint32_t n_inst;
     int precision;     // POTG_FP64 / POTG_MIXED / POTG_MIXED_GROUP
     int any_spheroid;  // some instance has the analytic spheroid grain
+    uint32_t n_lone64; // instances with lone64
     int count;         // step walks keep the interaction counters (potg_set_counting)
     int key_levels;    // digits carried by a sort key
     int key_bits;      // bits of the key that are sorted

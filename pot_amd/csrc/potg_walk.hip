@@ -57,7 +57,19 @@ struct WalkIO {
     const InstState* S;
     const double* dip64;   // record dipoles (DIPOLES instances), else null
     const float4* dip32;
+    // the targets of every instance (PICK_ALL), or of those that the float32
+    // or the float64 walk gives a wavefront each (InstParams::lone32, lone64)
+    // or 64 to one
+    int32_t pick;
 };
+enum { PICK_ALL = 0, PICK_LONE = 1, PICK_SHARED = 2, PICK_F64 = 4 };
+
+__device__ inline bool picked(const InstParams& p, int32_t pick)
+{
+    if (pick == PICK_ALL) return true;
+    const bool lone = ((pick & PICK_F64) ? p.lone64 : p.lone32) != 0;
+    return lone == ((pick & PICK_LONE) != 0);
+}
 
 __device__ inline void kahan_add(float& s, float& c, float v)
 {
@@ -101,6 +113,7 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
         if (i == NONE) return false;  // the gap before the next instance's targets
         self = i;
         inst = st.inst[i];
+        if (!picked(P[inst], io.pick)) return false;
         if (P[inst].integrator == 0) {
             const double dts = P[inst].dt * (double)P[inst].tss[st.spec[i]];
             tx = st.x[i] + (0.5 * dts) * st.vx[i];
@@ -114,6 +127,7 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
     } else if (MODE == MODE_EPE) {
         self = k;
         inst = st.inst[k];
+        if (!picked(P[inst], io.pick)) return false;
         const int sp = st.spec[k];
         // Boris half-drifted the stepped particles in place; the other
         // integrators' state already holds the intermediate state
@@ -133,15 +147,44 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
     return true;
 }
 
-// ---- float64 walk (field or potential) --------------------------------
+// 1 / sqrt(r2) to the last bits: the hardware's value (relative error below
+// 2^-23), then (1 - e)^(-1/2) = 1 + e/2 + 3/8 e^2 + O(e^3), e = 1 - r2 r^2
+__device__ inline double rsqrt64(double r2)
+{
+    const double r = __builtin_amdgcn_rsq(r2);
+    const double e = __builtin_fma(-r2 * r, r, 1.0);
+    return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
+}
+
+__device__ inline bool lane_of(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// ---- float64 walk, 64 targets per wavefront (field or potential) --------
+//
+// The order of k_walk32s (below): a child range is swept whole -- its leaves,
+// then every cell, each lane taking the cells its own target accepts -- and
+// the wavefront then descends into the opened cells, youngest first, the
+// range waiting on the stack.  The opening test is the reference's float64
+// expression, so the interaction sets are the reference's exactly.  The
+// range is staged in LDS and read back as broadcasts; lane sets are scalar
+// masks; 1 / r is the hardware's reciprocal square root refined to float64.
+// Bound by the float64 vector unit (about 34 issue slots a cell with its
+// dipole) and, next to it, by the LDS broadcasts (64 B a child for 64 lanes).
+// 500001 particles, DIPOLES, theta 0.14, prolate grain: 52.5 ms with lane
+// reads for the broadcasts and a square root and a division an interaction.
+struct Staged64 {
+    double cx, cy, cz, size2, q, px, py, pz;
+    uint32_t first, cnt, part, pad;
+};
+
 template <int MODE, int KIND, bool DIP, bool COUNT>
 __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P, Globals* g,
                                                 PState st, const NodeRec64* __restrict__ rec,
                                                 WalkIO io)
 {
     __shared__ uint32_t s_first[NW][STK];
-    __shared__ uint32_t s_cnt[NW][STK];
+    __shared__ uint32_t s_open[NW][STK];  // opened cells still to descend
     __shared__ uint64_t s_mask[NW][STK];
+    __shared__ Staged64 s_rec[NW][8];
     const int wv = threadIdx.x / WAVE;
     const uint32_t lane = __lane_id();
     const uint32_t ntg = (MODE == MODE_STEP) ? *io.n_targets_dev : io.n_pts;
@@ -156,17 +199,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
         uint32_t inst, self;
         double tx, ty, tz;
         const bool valid = load_target<MODE>(P, st, io, k, ntg, inst, self, tx, ty, tz);
-        const double theta2 = P[inst].theta2, soft2 = P[inst].soft2;
-        double ex = 0.0, ey = 0.0, ez = 0.0, ph = 0.0;
-        if (valid) {
-            if (io.acc && KIND == KIND_FIELD) {
-                ex = io.out[3 * k];
-                ey = io.out[3 * k + 1];
-                ez = io.out[3 * k + 2];
-            } else if (io.acc) {
-                ph = io.out[k];
-            }
-        }
+        double ex = 0.0, ey = 0.0, ez = 0.0;  // the sums (ex: a potential's)
         uint32_t ncell = 0, nleaf = 0, nopen = 0;
 
         uint64_t pending = ballot(valid);
@@ -175,146 +208,171 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
             const uint32_t gi = rfl(__shfl(inst, lead, WAVE));
             const uint64_t grp = rfl64(ballot(valid && inst == gi));
             pending &= ~grp;
+            if (rfl(P[gi].tree_n) == 0u) continue;  // no nodes
+            const double theta2 = P[gi].theta2, soft2 = P[gi].soft2;
             const bool dip = DIP && P[gi].dipoles && io.dip64;
+            // the range to sweep next: the root's
             uint32_t tf = gi, tc = 1;
             uint64_t tm = grp;
             int sp = 0;
             uint32_t loads = 0;
             for (;;) {
-                if (tc == 0) {
-                    if (sp == 0) break;
-                    --sp;
-                    tf = rfl(s_first[wv][sp]);
-                    tc = rfl(s_cnt[wv][sp]);
-                    tm = rfl64(s_mask[wv][sp]);
-                }
-                if (++loads > io.n_rec || tc > 8) {
+                if (++loads > io.n_rec || tc - 1u > 7u) {
                     raise_err(g, tc > 8 ? KERR_CAPACITY : KERR_DEPTH, tf);
                     break;
                 }
                 tot_pops++;
-                // one load for the whole range: lane j holds child j
-                NodeRec64 mine;
-                double mpx = 0.0, mpy = 0.0, mpz = 0.0;
-                if (lane < tc) mine = rec[tf + lane];
-                else mine = NodeRec64{0.0, 0.0, 0.0, 0.0, 0, 0, 0, 0};
-                if (dip && lane < tc) {
-                    mpx = io.dip64[3 * (size_t)(tf + lane)];
-                    mpy = io.dip64[3 * (size_t)(tf + lane) + 1];
-                    mpz = io.dip64[3 * (size_t)(tf + lane) + 2];
-                }
-                const bool act = (tm >> lane) & 1ull;
-                uint32_t next_first = 0, next_cnt = 0;
-                uint64_t next_mask = 0;
-                int j = (int)tc - 1;
-                for (; j >= 0; j--) {
-                    const double cx = bcast_d(mine.cx, j), cy = bcast_d(mine.cy, j),
-                                 cz = bcast_d(mine.cz, j);
-                    const uint32_t cnt = bcast_u(mine.cnt, j);
-                    const int q = (int)bcast_u((uint32_t)mine.q, j);
-                    bool open = false;
-                    if (act) {
-                        const double dx = tx - cx, dy = ty - cy, dz = tz - cz;
-                        const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
-                        if (cnt == LEAF) {
-                            if (KIND == KIND_FIELD) {
-                                if (bcast_u(mine.part, j) != self) {
-                                    if (d2 != 0.0) {
-                                        const double dd2 = d2 + soft2;
-                                        const double dist = sqrt(dd2);
-                                        const double es = (QE * q) / ((K4PE0 * dd2) * dist);
-                                        ex += es * dx;
-                                        ey += es * dy;
-                                        ez += es * dz;
-                                        nleaf++;
-                                    } else {
-                                        raise_err(g, KERR_COINCIDENT, self);
-                                    }
-                                }
-                            } else if (KIND == KIND_PHI || bcast_u(mine.part, j) != self) {
-                                ph += (QE * q) / (K4PE0 * sqrt(d2 + soft2));
-                                nleaf++;
-                            }
-                        } else if (bcast_d(mine.size2, j) < theta2 * d2) {
-                            // DIPOLES accepts every cell holding charge, net
-                            // or not (pot.c:1732-1736); internal records
-                            // carry |q| in `part`
-                            if (dip ? bcast_u(mine.part, j) != 0 : q != 0) {
-                                if (dip) {
-                                    const double px = bcast_d(mpx, j), py = bcast_d(mpy, j),
-                                                 pz = bcast_d(mpz, j);
-                                    const double dist = sqrt(d2);
-                                    if (KIND == KIND_FIELD) {
-                                        // pot.c:1738-1745
-                                        const double es = QE / ((K4PE0 * d2) * dist);
-                                        const double rpd2 = ((dx * px) + (dy * py) + (dz * pz)) / d2;
-                                        ex += es * ((q * dx) - px + ((3 * dx) * rpd2));
-                                        ey += es * ((q * dy) - py + ((3 * dy) * rpd2));
-                                        ez += es * ((q * dz) - pz + ((3 * dz) * rpd2));
-                                    } else {
-                                        const double rdp = (dx * px) + (dy * py) + (dz * pz);
-                                        const double t = (q / dist) + (rdp / (dist * d2));
-                                        // phi_at (pot.c:1862) and phi_particle_feels
-                                        // (pot.c:1969) group the constants differently
-                                        if (KIND == KIND_PHI) ph += (QE / K4PE0) * t;
-                                        else ph += (QE * t) / K4PE0;
-                                    }
-                                } else if (KIND == KIND_FIELD) {
-                                    const double dist = sqrt(d2);
-                                    double es = QE / ((K4PE0 * d2) * dist);
-                                    es *= q;
-                                    ex += es * dx;
-                                    ey += es * dy;
-                                    ez += es * dz;
-                                } else {
-                                    ph += (QE * q) / (K4PE0 * sqrt(d2));
-                                }
-                                ncell++;
-                            }
-                        } else {
-                            open = cnt != 0;
+                uint32_t lm, chg;
+                {
+                    const bool in = lane < tc;
+                    const uint32_t w = tf + (in ? lane : 0u);
+                    const NodeRec64 r = rec[w];
+                    if (in) {
+                        Staged64& d = s_rec[wv][lane];
+                        d.cx = r.cx;
+                        d.cy = r.cy;
+                        d.cz = r.cz;
+                        d.size2 = r.size2;
+                        d.q = (double)r.q;
+                        d.first = r.first;
+                        d.cnt = r.cnt;
+                        d.part = r.part;
+                        if (DIP && dip) {
+                            d.px = io.dip64[3 * (size_t)w];
+                            d.py = io.dip64[3 * (size_t)w + 1];
+                            d.pz = io.dip64[3 * (size_t)w + 2];
                         }
                     }
-                    const uint64_t om = rfl64(ballot(open));
-                    if (om) {
-                        if (open) nopen++;
-                        next_first = bcast_u(mine.first, j);
-                        next_cnt = cnt;
-                        next_mask = om;
-                        break;
+                    const uint32_t inm = (1u << tc) - 1u;
+                    lm = (uint32_t)ballot(r.cnt == LEAF) & inm;
+                    // DIPOLES takes every cell holding charge, net or not
+                    // (pot.c:1732-1736); internal records carry |q| in `part`
+                    chg = (uint32_t)ballot((DIP && dip) ? r.part != 0u : r.q != 0) & inm;
+                }
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t all = (1u << tc) - 1u;
+                const uint32_t lv = all & lm, cl = all & ~lm;
+                for (uint32_t m = lv; m; m &= m - 1u) {
+                    const Staged64& r = s_rec[wv][__builtin_ctz(m)];
+                    const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
+                    const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
+                    uint64_t m_use = tm;
+                    // a target skips its own leaf (pot.c:1787)
+                    if (KIND != KIND_PHI) m_use &= ~ballot(r.part == self);
+                    if (KIND == KIND_FIELD) {
+                        const uint64_t m_hit = m_use & ballot(d2 == 0.0);
+                        if (m_hit) {
+                            if (lane_of(m_hit)) raise_err(g, KERR_COINCIDENT, self);
+                            m_use &= ~m_hit;
+                        }
                     }
+                    const double r2 = d2 + soft2;
+                    double inv = rsqrt64(r2);
+                    if (KIND != KIND_FIELD && r2 == 0.0) inv = __builtin_inf();
+                    inv = lane_of(m_use) ? inv : 0.0;
+                    if (KIND == KIND_FIELD) {
+                        const double ca = r.q * (inv * inv * inv);
+                        ex = __builtin_fma(ca, dx, ex);
+                        ey = __builtin_fma(ca, dy, ey);
+                        ez = __builtin_fma(ca, dz, ez);
+                    } else {
+                        ex = __builtin_fma(r.q, inv, ex);
+                    }
+                    if (COUNT) nleaf += lane_of(m_use) ? 1u : 0u;
                 }
-                if (j < 0) {
-                    tc = 0;
-                    continue;
+                uint32_t opened = 0;
+                uint64_t om = 0;  // the lanes that open the youngest opened cell
+                for (uint32_t m = cl; m;) {
+                    const uint32_t j = 31u - (uint32_t)__builtin_clz(m);
+                    m &= ~(1u << j);
+                    const Staged64& r = s_rec[wv][j];
+                    const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
+                    const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
+                    const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
+                    const uint64_t m_use = tm & m_acc, m_open = tm & ~m_acc;
+                    if (m_open) {
+                        if (COUNT) nopen += lane_of(m_open) ? 1u : 0u;
+                        if (!opened) om = m_open;
+                        opened |= 1u << j;
+                    }
+                    if (!m_use) continue;
+                    const double inv = lane_of(m_use) ? rsqrt64(d2) : 0.0;
+                    const double inv2 = inv * inv, inv3 = inv2 * inv;
+                    if (DIP && dip) {
+                        const double rdp =
+                            __builtin_fma(dx, r.px, __builtin_fma(dy, r.py, dz * r.pz));
+                        if (KIND == KIND_FIELD) {
+                            // pot.c:1738-1745: q d / r^3 - p / r^3 + 3 (d.p) d / r^5
+                            const double ca = __builtin_fma(3.0, rdp * inv2, r.q);
+                            ex = __builtin_fma(inv3, __builtin_fma(ca, dx, -r.px), ex);
+                            ey = __builtin_fma(inv3, __builtin_fma(ca, dy, -r.py), ey);
+                            ez = __builtin_fma(inv3, __builtin_fma(ca, dz, -r.pz), ez);
+                        } else {
+                            ex = __builtin_fma(inv3, rdp, __builtin_fma(r.q, inv, ex));
+                        }
+                    } else if (KIND == KIND_FIELD) {
+                        const double ca = r.q * inv3;
+                        ex = __builtin_fma(ca, dx, ex);
+                        ey = __builtin_fma(ca, dy, ey);
+                        ez = __builtin_fma(ca, dz, ez);
+                    } else {
+                        ex = __builtin_fma(r.q, inv, ex);
+                    }
+                    if (COUNT && ((chg >> j) & 1u)) ncell += lane_of(m_use) ? 1u : 0u;
                 }
-                // descend into child j; its elder siblings wait on the stack
-                if (next_first <= tf + (uint32_t)j || next_first + next_cnt > io.n_rec) {
+                uint32_t j = 0, next_first = 0, next_cnt = 0;
+                if (opened) {
+                    j = 31u - (uint32_t)__builtin_clz(opened);
+                    opened &= ~(1u << j);
+                    next_first = rfl(s_rec[wv][j].first);
+                    next_cnt = rfl(s_rec[wv][j].cnt);
+                } else {
+                    // the next opened cell of a range waiting on the stack, and
+                    // the lanes that open it, found again by the same test
+                    while (sp > 0 && om == 0) {
+                        uint32_t rest = rfl(s_open[wv][sp - 1]);
+                        tf = rfl(s_first[wv][sp - 1]);
+                        tm = rfl64(s_mask[wv][sp - 1]);
+                        j = 31u - (uint32_t)__builtin_clz(rest);
+                        rest &= ~(1u << j);
+                        if (rest) s_open[wv][sp - 1] = rest;
+                        else --sp;
+                        const NodeRec64 r = rec[tf + j];
+                        const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
+                        const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
+                        om = tm & ballot(theta2 * d2 <= r.size2);
+                        next_first = rfl(r.first);
+                        next_cnt = rfl(r.cnt);
+                    }
+                    if (om == 0) break;  // stack empty: the instance group is done
+                }
+                if (next_first <= tf + j || next_cnt - 1u > 7u || next_first + next_cnt > io.n_rec) {
                     raise_err(g, KERR_CAPACITY, tf + j);
                     break;
                 }
-                if (j > 0) {
+                if (opened) {
                     if (sp >= STK) {
                         raise_err(g, KERR_DEPTH, tf);
                         break;
                     }
                     s_first[wv][sp] = tf;
-                    s_cnt[wv][sp] = (uint32_t)j;
+                    s_open[wv][sp] = opened;
                     s_mask[wv][sp] = tm;
                     sp++;
                 }
                 tf = next_first;
                 tc = next_cnt;
-                tm = next_mask;
+                tm = om;
             }
         }
         if (valid) {
+            const double K = QE / K4PE0;
             if (KIND == KIND_FIELD) {
-                io.out[3 * k] = ex;
-                io.out[3 * k + 1] = ey;
-                io.out[3 * k + 2] = ez;
+                io.out[3 * k] = (io.acc ? io.out[3 * k] : 0.0) + K * ex;
+                io.out[3 * k + 1] = (io.acc ? io.out[3 * k + 1] : 0.0) + K * ey;
+                io.out[3 * k + 2] = (io.acc ? io.out[3 * k + 2] : 0.0) + K * ez;
             } else {
-                io.out[k] = ph;
+                io.out[k] = (io.acc ? io.out[k] : 0.0) + K * ex;
             }
         }
         tot_cell += ncell;
@@ -922,15 +980,6 @@ constexpr int NS1 = 632;
 // more), above it one, depth first, which adds at most 7 a level
 constexpr int SP1_WIDE = NS1 - 7 * MAXD - 56;
 
-// 1 / sqrt(r2) to the last bits: the hardware's value (relative error below
-// 2^-23), then (1 - e)^(-1/2) = 1 + e/2 + 3/8 e^2 + O(e^3), e = 1 - r2 r^2
-__device__ inline double rsqrt64(double r2)
-{
-    const double r = __builtin_amdgcn_rsq(r2);
-    const double e = __builtin_fma(-r2 * r, r, 1.0);
-    return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
-}
-
 // row_shr 1, 2, 4, 8 added up: lane 15 of each 16-lane row holds its sum
 template <int CTRL>
 __device__ inline double dpp_add(double v)
@@ -970,8 +1019,6 @@ __device__ inline uint32_t wave_sum_u(uint32_t v)
     for (int d = 1; d < WAVE; d <<= 1) v += __shfl_xor(v, d, WAVE);
     return v;
 }
-__device__ inline bool lane_of(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
-
 template <bool F64>
 struct Walk1Rec { using type = NodeRec32; };
 template <>
@@ -1792,11 +1839,27 @@ static void launch_walk64c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
         k_walk64<MODE, KIND, false, COUNT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, b.rec64, io);
 }
 
-template <int MODE, int KIND>
-static void launch_walk64(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
+// float64 walk: the instances that walk alone and those that walk together,
+// each by its kernel; `blocks` for the latter
+template <int MODE, int KIND, bool COUNT>
+static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream_t s)
 {
-    if (b.count) launch_walk64c<MODE, KIND, true>(b, blocks, io, s);
-    else launch_walk64c<MODE, KIND, false>(b, blocks, io, s);
+    const bool all = b.n_lone64 == b.n_inst;
+    if (b.n_lone64) {
+        io.pick = all ? PICK_ALL : PICK_LONE | PICK_F64;
+        launch_walk1<true, MODE, KIND, COUNT>(b, n, io, s);
+    }
+    if (!all) {
+        io.pick = b.n_lone64 ? PICK_SHARED | PICK_F64 : PICK_ALL;
+        launch_walk64c<MODE, KIND, COUNT>(b, blocks, io, s);
+    }
+}
+
+template <int MODE, int KIND>
+static void launch_walk64(Bufs& b, int blocks, uint32_t n, const WalkIO& io, hipStream_t s)
+{
+    if (b.count) launch_walk64p<MODE, KIND, true>(b, blocks, n, io, s);
+    else launch_walk64p<MODE, KIND, false>(b, blocks, n, io, s);
 }
 
 void launch_walk(Bufs& b, hipStream_t s)
@@ -1805,7 +1868,7 @@ void launch_walk(Bufs& b, hipStream_t s)
     if (b.precision)
         launch_walk32<MODE_STEP>(b, (int)b.walk_blocks, io, s);
     else
-        launch_walk64<MODE_STEP, KIND_FIELD>(b, (int)b.walk_blocks, io, s);
+        launch_walk64<MODE_STEP, KIND_FIELD>(b, (int)b.walk_blocks, b.t_cap, io, s);
 }
 
 void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s)
@@ -1887,7 +1950,7 @@ void launch_epe(Bufs& b, hipStream_t s)
     const uint32_t nb = (b.n_total + BT - 1) / BT;
     const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
     k_grain_init<MODE_EPE, KIND_EPE><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-    launch_walk64<MODE_EPE, KIND_EPE>(b, blocks, io, s);
+    launch_walk64<MODE_EPE, KIND_EPE>(b, blocks, b.n_total, io, s);
     k_epe_partial<<<dim3(EPE_BLOCKS, b.n_inst), BT, 0, s>>>(b.P, b.st, b.phi, b.epe_part);
 }
 
