@@ -151,17 +151,17 @@ typedef struct potg_stats_t {
    64-target tiles per CU (half the particles are targets): the float32
    walk sweeps whole ranges with 64 targets per wavefront on 8 blocks per CU
    from 16 tiles per CU (about 0.5M particles), on 2 blocks per CU from 1
-   tile per CU, and below that takes 8 targets per wavefront, one after the
-   other; the float64 walk takes 64 targets on 8 blocks per CU from 16
-   tiles per CU, 4 below. */
+   tile per CU, and below that takes 8 targets per wavefront on 2 blocks
+   per CU; the float64 walk takes 8 blocks per CU from 16 tiles per CU, 4
+   below.  They concern step walks (point queries follow a group of 16 or
+   variant 0 only) and, of the float64 ones, those of instances with 64
+   targets per wavefront: an instance whose opening angle is large for its
+   size, or with less than half a million particles, is walked 2 by 2. */
 typedef struct potg_tuning {
-    uint32_t walk_blocks; /* blocks (4 wavefronts each) of the persistent walk;
-                             not used by a walk of 8 targets per wavefront */
+    uint32_t walk_blocks; /* blocks (4 wavefronts each) of the persistent walk */
     uint32_t group;       /* float32 walk: targets per wavefront, 8, 16 or 64;
-                             with 8 (at most: fewer in a small context) they are
-                             walked one after the other, 64 nodes at once; with
-                             16 the wavefront evaluates 4 children per target
-                             at once */
+                             with 8 or 16 the wavefront evaluates 8 or 4
+                             children per target at once */
     uint32_t variant;     /* float32 walk with 64 targets: 0 visits a range's
                              cells until some lanes open one, 1 sweeps every
                              range whole before descending */

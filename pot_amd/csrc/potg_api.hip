@@ -190,20 +190,25 @@ void fill_params(InstParams& p, const potg_config& k)
     for (int s = 0; s < 3; s++) p.first_idx[s] = NONE;
 }
 
-// Whether the float64 walk gives each target a wavefront of its own (k_walk1)
-// or 64 to one (k_walk64).  Alone, no lane works for another's target, but
-// every node comes through the L1 once per target; 64 neighbours share the
-// loads, and the more of their nodes the smaller theta, but 64-target tiles
-// are too few to fill a device below a few hundred thousand particles.
-// Step walk, ms, alone / together: 150k particles theta 0.8 0.10 / 0.62, theta
-// 0.14 DIPOLES 5.7 / 15.5; 500k theta 0.3 3.8 / 5.6, 0.2 11.9 / 13.1, 0.14
-// 33.9 / 26.2 (all DIPOLES); 2M theta 0.5 2.9 / 4.6, 0.3 10.9 / 12.0, 0.14
-// DIPOLES 204 / 77.  By an instance's own values, so that its walk is the same
-// alone and in a batch.
+// Whether an instance's float64 walk has 2 targets a wavefront (k_walk1) or 64
+// (k_walk64).  With few, hardly a lane works for another's target; 64 share
+// every node's load and its instructions, the better the smaller theta,
+// since neighbours' sets then differ less, and the larger the tree, whose
+// nodes a few targets fetch from further away -- but a tile of 64 is a long
+// walk, too few of which keep a device below half a million particles busy to
+// the end.  Step walk, ms, 2 / 64 targets, for DIPOLES (monopoles cross over
+// about 0.03 lower in theta):
+//   theta  150k       500k       1M         2M
+//   0.14   4.5/15.6   24.5/27.1  60/43      146/79
+//   0.20   2.0/8.2    9.1/13.7   21.5/20.5  50/38
+//   0.25   1.2/5.5    4.9/8.6    11.0/12.9  25/24
+//   0.30   0.8/3.9    3.0/5.9    6.4/8.8    14/16
+// so the crossing is put at theta = c + 0.05 log2(N / 1M).  By an instance's
+// own values, so that its walk is the same alone and in a batch.
 int lone64_rule(const InstParams& p)
 {
-    const double theta = sqrt(p.theta2);
-    return theta >= 0.25 || (theta >= 0.17 && p.tree_n < 800000u) || p.tree_n < 250000u;
+    if (p.tree_n < 500000u) return 1;
+    return sqrt(p.theta2) >= (p.dipoles ? 0.21 : 0.18) + 0.05 * log2((double)p.tree_n / 1e6);
 }
 
 // chi_b sampling point of the one worker (measure_chi_b, pot.c:2257-2275)

@@ -74,7 +74,7 @@ struct InstParams {
     int32_t integrator;    // POTG_BORIS / POTG_VERLET / POTG_EULER_RICHARDSON
     int32_t out_bounce;    // OUT_BOUNCE: bounce off the wall
     double bounce_coe;     // its coefficient of restitution
-    int32_t lone32, lone64; // the float32 / float64 walk gives each target a wavefront
+    int32_t lone64;        // the float64 walk has few targets a wavefront
 };
 
 // Mutable per-instance state on the device.

@@ -57,18 +57,15 @@ struct WalkIO {
     const InstState* S;
     const double* dip64;   // record dipoles (DIPOLES instances), else null
     const float4* dip32;
-    // the targets of every instance (PICK_ALL), or of those that the float32
-    // or the float64 walk gives a wavefront each (InstParams::lone32, lone64)
-    // or 64 to one
+    // the targets of every instance (PICK_ALL), or of those whose float64 walk
+    // has few targets a wavefront (InstParams::lone64), or 64
     int32_t pick;
 };
-enum { PICK_ALL = 0, PICK_LONE = 1, PICK_SHARED = 2, PICK_F64 = 4 };
+enum { PICK_ALL = 0, PICK_LONE = 1, PICK_SHARED = 2 };
 
 __device__ inline bool picked(const InstParams& p, int32_t pick)
 {
-    if (pick == PICK_ALL) return true;
-    const bool lone = ((pick & PICK_F64) ? p.lone64 : p.lone32) != 0;
-    return lone == ((pick & PICK_LONE) != 0);
+    return pick == PICK_ALL || (p.lone64 != 0) == (pick == PICK_LONE);
 }
 
 __device__ inline void kahan_add(float& s, float& c, float v)
@@ -950,30 +947,43 @@ __global__ __launch_bounds__(BT) void k_walk32s(const InstParams* __restrict__ P
     }
 }
 
-// ---- one target per wavefront ---------------------------------------------
+// ---- 1 or 2 targets per wavefront, 64 nodes at once -------------------------
 //
-// The 64 lanes of a wavefront test 64 nodes against one target: up to 8
-// child ranges are taken off an LDS stack at once, lane = 8 range + child,
-// and the ranges of the children that the target opens are pushed back.
-// The interaction set is the reference's, and no lane works for another
-// target's: a wavefront that walks for several targets steps through the
-// union of their sets, which for 64 neighbours is 2.3 (theta 0.5, 2M
-// particles) to 4 times one target's, and for scattered points many times it.
-// The loads are 32- or 48-byte gathers from L2, 8 contiguous records a range.
-// Step walk, mixed, theta 0.5: 16k particles 0.36 (8 targets against 8
-// children at once) -> 0.028 ms.  The force at 65536 scattered points of 1M
+// Point queries of both precisions, the potential-energy walk and, where few
+// targets a wavefront are the faster shape (lone64), the float64 step walk.
+// (The float32 step walks keep k_walkg's and k_walk32s's order of summation.)
+//
+// The 64 lanes of a wavefront hold 64 nodes: up to 8 child ranges are taken
+// off an LDS stack at once, lane = 8 range + child, the nodes are tested
+// against T targets one after the other, and the ranges of the children that
+// some of them open are pushed back with a bit for each target that does.
+// The interaction sets are the reference's.  A wavefront that walks for 64
+// targets steps through the union of their sets, 2.3 (theta 0.5, 2M
+// particles) to 4 times one target's for neighbours and many times it for
+// scattered points; the union of 2 is 1.1 times one's, and lanes idle only
+// past the end of a range.
+//
+// The loads are gathers of 32- or 48-byte records, 8 contiguous ones a range,
+// nearly all from L2.  With one target a wavefront their lines are the bound;
+// two use a line twice and share the stack's instructions (float64 step walk,
+// 2M particles, theta 0.5: 3.10 -> 2.62 ms, 9.0 with 64 targets, readlane
+// broadcasts and divisions; 4 targets run out of registers: 2.80).  Point
+// queries take one, since points come in the caller's order, and so does the
+// potential-energy walk, whose pairs would depend on where an instance's
+// slots start in a batch.  The force at 65536 scattered points of 1M
 // particles with its tree build 12.6 -> 3.4 ms, the potential at 2200 grid
-// points of 150k particles 2.37 -> 0.08 ms (64 points shared a traversal).
+// points of 150k particles 2.37 -> 0.08 ms against 64 points sharing a
+// traversal.
 //
-// Targets of a wavefront (per_wave at most 8) are read together, lane by
-// lane, and walked one after the other.  Neighbouring blocks, which the
+// Targets of a wavefront (per_wave, a power of two from T to 8) are read
+// together, lane by lane, and walked T by T.  Neighbouring blocks, which the
 // hardware deals to the 8 XCDs in turn, take targets from 8 separate
 // stretches of the list, so that each XCD's L2 holds one region's nodes.
 //
-// float32: each lane sums its own interactions, flushed every 4 passes into a
+// float32: each lane sums its own interactions, flushed every 8 passes into a
 // compensated sum; the lanes' sums are added in float64, in a fixed order.
 // float64: plain float64 sums; 1 / r from the hardware's reciprocal square
-// root, refined.  Every result depends on its target and the tree alone.
+// root, refined.  A result depends on its group of T targets and the tree.
 constexpr uint32_t XCDS = 8;
 constexpr int NS1 = 632;
 // below this the stack takes 8 ranges at a time (which leaves at most 56
@@ -1024,8 +1034,8 @@ struct Walk1Rec { using type = NodeRec32; };
 template <>
 struct Walk1Rec<true> { using type = NodeRec64; };
 
-template <bool F64, int MODE, int KIND, bool DIP, bool COUNT>
-__global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, Globals* g,
+template <int T, bool F64, int MODE, int KIND, bool DIP, bool COUNT>
+__global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ P, Globals* g,
                                               PState st,
                                               const typename Walk1Rec<F64>::type* __restrict__ rec,
                                               WalkIO io, uint32_t per_wave)
@@ -1034,7 +1044,8 @@ __global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, 
     // float32: a range's first record counted in 16-byte units (2 n_rec stays
     // below 2^32 for any context that fits the device), an address of one add
     constexpr uint32_t U = F64 ? 1 : 2;
-    // a range's first record (times U) and its count; below the stack 8
+    // a range's first record (times U), its count and, with T > 1, the targets
+    // that opened it (a bit each from bit 8); below the stack 8
     // entries without children, so that a pass always reads 8
     __shared__ uint2 s_mem[NW][8 + NS1];
     const int wv = threadIdx.x / WAVE;
@@ -1066,36 +1077,58 @@ __global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, 
             l_fz = (float)((l_z - p.R) * p.invR);
             l_soft2 = (float)(p.soft2 * p.invR * p.invR);
         }
-        for (uint64_t todo = ballot(valid); todo; todo &= todo - 1u) {
-            const uint32_t src = (uint32_t)__builtin_ctzll(todo);
-            const uint32_t k = k0 + src;
-            const uint32_t gi = bcast_u(l_inst, src), self = bcast_u(l_self, src);
+        uint64_t todo = ballot(valid);
+        while (todo) {
+            // T targets of one instance
+            const uint32_t src0 = (uint32_t)__builtin_ctzll(todo);
+            const uint32_t gi = bcast_u(l_inst, src0);
+            uint64_t same = T == 1 ? todo : todo & ballot(l_inst == gi);
+            uint32_t src[T], self[T], have = 0;
             const InstParams& p = P[gi];
             const bool dip = DIP && p.dipoles && (F64 ? (const void*)io.dip64 : (const void*)io.dip32);
-            float tx = 0.f, ty = 0.f, tz = 0.f, soft2f = 0.f;
-            double dtx = 0.0, dty = 0.0, dtz = 0.0, theta2 = 0.0, soft2 = 0.0;
+            float tx[T], ty[T], tz[T], soft2f = 0.f;
+            double dtx[T], dty[T], dtz[T], theta2 = 0.0, soft2 = 0.0;
+#pragma unroll
+            for (int i = 0; i < T; i++) {
+                // a missing target repeats the first and takes part in nothing
+                src[i] = same ? (uint32_t)__builtin_ctzll(same) : src0;
+                have |= same ? 1u << i : 0u;
+                todo &= ~(1ull << src[i]);
+                same &= same - 1u;
+                self[i] = bcast_u(l_self, src[i]);
+                if constexpr (F64) {
+                    dtx[i] = bcast_d(l_x, src[i]);
+                    dty[i] = bcast_d(l_y, src[i]);
+                    dtz[i] = bcast_d(l_z, src[i]);
+                } else {
+                    tx[i] = bcast_f(l_fx, src[i]);
+                    ty[i] = bcast_f(l_fy, src[i]);
+                    tz[i] = bcast_f(l_fz, src[i]);
+                }
+            }
             if constexpr (F64) {
-                dtx = bcast_d(l_x, src);
-                dty = bcast_d(l_y, src);
-                dtz = bcast_d(l_z, src);
                 theta2 = p.theta2;
                 soft2 = p.soft2;
             } else {
-                tx = bcast_f(l_fx, src);
-                ty = bcast_f(l_fy, src);
-                tz = bcast_f(l_fz, src);
-                soft2f = bcast_f(l_soft2, src);
+                soft2f = bcast_f(l_soft2, src0);
             }
-            double ex = 0.0, ey = 0.0, ez = 0.0;  // float64: the sums (ex: a potential's)
-            float fx = 0.f, fy = 0.f, fz = 0.f, kx = 0.f, ky = 0.f, kz = 0.f;
-            uint32_t ncell = 0, nleaf = 0, nopen = 0, loads = 0;
+            double ex[T], ey[T], ez[T];  // float64: the sums (ex: a potential's)
+            float fx[T], fy[T], fz[T], kx[T], ky[T], kz[T];
+#pragma unroll
+            for (int i = 0; i < T; i++) {
+                ex[i] = ey[i] = ez[i] = 0.0;
+                fx[i] = fy[i] = fz[i] = kx[i] = ky[i] = kz[i] = 0.f;
+            }
+            uint32_t ncell[T] = {}, nleaf[T] = {}, nopen[T] = {}, loads = 0;
             // the root alone; an empty instance has no nodes
-            if (lane == 0) s_stk[0] = make_uint2(gi * U, 1u);
+            if (lane == 0) s_stk[0] = make_uint2(gi * U, 1u | (have << 8));
             __builtin_amdgcn_wave_barrier();
             int sp = rfl(p.tree_n) != 0u ? 1 : 0;
             while (sp > 0) {
-                float px = 0.f, py = 0.f, pz = 0.f;
-                for (int u = 0; u < 4 && sp > 0; u++) {
+                float px[T], py[T], pz[T];
+#pragma unroll
+                for (int i = 0; i < T; i++) px[i] = py[i] = pz[i] = 0.f;
+                for (int u = 0; u < 8 && sp > 0; u++) {
                     const bool wide = sp <= SP1_WIDE;
                     int take = wide ? (sp < 8 ? sp : 8) : 1;
                     asm("" : "+s"(take));
@@ -1103,8 +1136,8 @@ __global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, 
                     // read a record that is there and add nothing; lane sets
                     // are scalar masks
                     const uint2 en = s_top[sp];
-                    const uint64_t m_in = ballot(ci < en.y) & (wide ? ~0ull : 0xffull);
-                    const uint32_t w = en.x + (lane_of(m_in) ? ci * U : 0u);
+                    const uint64_t m_rng = ballot(ci < (en.y & 0xffu)) & (wide ? ~0ull : 0xffull);
+                    const uint32_t w = en.x + (lane_of(m_rng) ? ci * U : 0u);
                     const int base = sp - take;
                     loads += (uint32_t)take;
                     const uint32_t wr = w / U;
@@ -1112,88 +1145,108 @@ __global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, 
                     if constexpr (F64) r = rec[w];
                     else r = *(const Rec*)((const uint4*)rec + w);
                     const uint64_t m_leaf = ballot(r.cnt == LEAF);
-                    const uint64_t m_own = KIND == KIND_PHI ? 0ull : m_leaf & ballot(r.part == self);
-                    uint64_t m_use, m_open;
-                    if constexpr (F64) {
-                        const double dx = dtx - r.cx, dy = dty - r.cy, dz = dtz - r.cz;
-                        // the reference's opening test, in its operations
-                        const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
-                        const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
-                        m_use = m_in & (m_acc | m_leaf) & ~m_own;
-                        if (KIND == KIND_FIELD) {
-                            const uint64_t m_hit = m_use & m_leaf & ballot(d2 == 0.0);
-                            if (m_hit) {
-                                if (lane_of(m_hit)) raise_err(g, KERR_COINCIDENT, self);
-                                m_use &= ~m_hit;
-                            }
-                        }
-                        m_open = m_in & ~(m_acc | m_leaf);
-                        const bool use = lane_of(m_use);
-                        const double r2 = lane_of(m_leaf) ? d2 + soft2 : d2;
-                        double inv = rsqrt64(r2);
-                        if (KIND != KIND_FIELD && r2 == 0.0) inv = __builtin_inf();
-                        inv = use ? inv : 0.0;
-                        const double q = (double)r.q;
-                        if (KIND == KIND_FIELD) {
-                            const double inv2 = inv * inv, inv3 = inv2 * inv;
-                            if (DIP && dip) {
-                                // zero for a leaf
-                                const double* dp = io.dip64 + 3 * (size_t)wr;
-                                const double pdx = dp[0], pdy = dp[1], pdz = dp[2];
-                                const double rpd2 =
-                                    __builtin_fma(dx, pdx, __builtin_fma(dy, pdy, dz * pdz)) * inv2;
-                                const double ca = __builtin_fma(3.0, rpd2, q);
-                                ex = __builtin_fma(inv3, __builtin_fma(ca, dx, -pdx), ex);
-                                ey = __builtin_fma(inv3, __builtin_fma(ca, dy, -pdy), ey);
-                                ez = __builtin_fma(inv3, __builtin_fma(ca, dz, -pdz), ez);
-                            } else {
-                                const double ca = q * inv3;
-                                ex = __builtin_fma(ca, dx, ex);
-                                ey = __builtin_fma(ca, dy, ey);
-                                ez = __builtin_fma(ca, dz, ez);
-                            }
+                    const float soft = !F64 && lane_of(m_leaf) ? soft2f : 0.f;
+                    uint64_t m_open = 0;  // by any of the targets
+                    uint32_t y = r.cnt;
+                    float4 pd = make_float4(0.f, 0.f, 0.f, 0.f);
+                    double pdx = 0.0, pdy = 0.0, pdz = 0.0;  // zero for a leaf
+                    if (DIP && dip) {
+                        if constexpr (F64) {
+                            pdx = io.dip64[3 * (size_t)wr];
+                            pdy = io.dip64[3 * (size_t)wr + 1];
+                            pdz = io.dip64[3 * (size_t)wr + 2];
                         } else {
-                            double ph = q * inv;
-                            if (DIP && dip) {
-                                // zero for a leaf
-                                const double* dp = io.dip64 + 3 * (size_t)wr;
-                                const double rdp =
-                                    __builtin_fma(dx, dp[0], __builtin_fma(dy, dp[1], dz * dp[2]));
-                                if (!lane_of(m_leaf)) ph = __builtin_fma(rdp * inv, inv * inv, ph);
-                            }
-                            ex += use ? ph : 0.0;
-                        }
-                    } else {
-                        const float dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
-                        const float d2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-                        // a leaf's size2 is zero: a leaf at float32 distance
-                        // zero adds nothing
-                        const uint64_t m_acc = ballot(!(d2 <= r.size2));
-                        m_use = m_in & m_acc & ~m_own;
-                        m_open = m_in & ~(m_acc | m_leaf);
-                        const float r2 = d2 + (lane_of(m_leaf) ? soft2f : 0.f);
-                        const float inv = lane_of(m_use) ? __builtin_amdgcn_rsqf(r2) : 0.f;
-                        const float inv2 = inv * inv, inv3 = inv2 * inv;
-                        if (DIP && dip) {
-                            const float4 pd = io.dip32[wr];
-                            const float rpd2 =
-                                __builtin_fmaf(dx, pd.x, __builtin_fmaf(dy, pd.y, dz * pd.z)) * inv2;
-                            const float ca = __builtin_fmaf(3.f, rpd2, r.q);
-                            px = __builtin_fmaf(inv3, __builtin_fmaf(ca, dx, -pd.x), px);
-                            py = __builtin_fmaf(inv3, __builtin_fmaf(ca, dy, -pd.y), py);
-                            pz = __builtin_fmaf(inv3, __builtin_fmaf(ca, dz, -pd.z), pz);
-                        } else {
-                            const float ca = r.q * inv3;
-                            px = __builtin_fmaf(ca, dx, px);
-                            py = __builtin_fmaf(ca, dy, py);
-                            pz = __builtin_fmaf(ca, dz, pz);
+                            pd = io.dip32[wr];
                         }
                     }
-                    if (COUNT) {
-                        const uint64_t m_chg = ballot(dip ? r.part != 0u : r.q != 0);
-                        ncell += lane_of(m_use & ~m_leaf & m_chg) ? 1u : 0u;
-                        nleaf += lane_of(m_use & m_leaf) ? 1u : 0u;
-                        nopen += lane_of(m_open) ? 1u : 0u;
+#pragma unroll
+                    for (int i = 0; i < T; i++) {
+                        const uint64_t m_in = T == 1 ? m_rng : m_rng & ballot((en.y & (256u << i)) != 0u);
+                        const uint64_t m_own =
+                            KIND == KIND_PHI ? 0ull : m_leaf & ballot(r.part == self[i]);
+                        uint64_t m_use, m_op;
+                        if constexpr (F64) {
+                            const double dx = dtx[i] - r.cx, dy = dty[i] - r.cy, dz = dtz[i] - r.cz;
+                            // the reference's opening test, in its operations
+                            const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
+                            const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
+                            m_use = m_in & (m_acc | m_leaf) & ~m_own;
+                            if (KIND == KIND_FIELD) {
+                                const uint64_t m_hit = m_use & m_leaf & ballot(d2 == 0.0);
+                                if (m_hit) {
+                                    if (lane_of(m_hit)) raise_err(g, KERR_COINCIDENT, self[i]);
+                                    m_use &= ~m_hit;
+                                }
+                            }
+                            m_op = m_in & ~(m_acc | m_leaf);
+                            const bool use = lane_of(m_use);
+                            const double r2 = lane_of(m_leaf) ? d2 + soft2 : d2;
+                            double inv = rsqrt64(r2);
+                            if (KIND != KIND_FIELD && r2 == 0.0) inv = __builtin_inf();
+                            inv = use ? inv : 0.0;
+                            const double q = (double)r.q;
+                            if (KIND == KIND_FIELD) {
+                                const double inv2 = inv * inv, inv3 = inv2 * inv;
+                                if (DIP && dip) {
+                                    const double rpd2 =
+                                        __builtin_fma(dx, pdx, __builtin_fma(dy, pdy, dz * pdz)) * inv2;
+                                    const double ca = __builtin_fma(3.0, rpd2, q);
+                                    ex[i] = __builtin_fma(inv3, __builtin_fma(ca, dx, -pdx), ex[i]);
+                                    ey[i] = __builtin_fma(inv3, __builtin_fma(ca, dy, -pdy), ey[i]);
+                                    ez[i] = __builtin_fma(inv3, __builtin_fma(ca, dz, -pdz), ez[i]);
+                                } else {
+                                    const double ca = q * inv3;
+                                    ex[i] = __builtin_fma(ca, dx, ex[i]);
+                                    ey[i] = __builtin_fma(ca, dy, ey[i]);
+                                    ez[i] = __builtin_fma(ca, dz, ez[i]);
+                                }
+                            } else {
+                                double ph = q * inv;
+                                if (DIP && dip) {
+                                    const double rdp =
+                                        __builtin_fma(dx, pdx, __builtin_fma(dy, pdy, dz * pdz));
+                                    if (!lane_of(m_leaf)) ph = __builtin_fma(rdp * inv, inv * inv, ph);
+                                }
+                                ex[i] += use ? ph : 0.0;
+                            }
+                        } else {
+                            const float dx = tx[i] - r.cx, dy = ty[i] - r.cy, dz = tz[i] - r.cz;
+                            // softened for leaves; for cells the softening is
+                            // zero and d2 the plain squared distance.  A leaf's
+                            // size2 is zero: unsoftened at float32 distance
+                            // zero it is not taken, softened it adds zero
+                            const float d2 =
+                                __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, soft)));
+                            const uint64_t m_acc = ballot(!(d2 <= r.size2));
+                            m_use = m_in & m_acc & ~m_own;
+                            m_op = m_in & ~(m_acc | m_leaf);
+                            const float inv = lane_of(m_use) ? __builtin_amdgcn_rsqf(d2) : 0.f;
+                            const float inv2 = inv * inv, inv3 = inv2 * inv;
+                            if (DIP && dip) {
+                                const float rpd2 =
+                                    __builtin_fmaf(dx, pd.x, __builtin_fmaf(dy, pd.y, dz * pd.z)) * inv2;
+                                const float ca = __builtin_fmaf(3.f, rpd2, r.q);
+                                px[i] = __builtin_fmaf(inv3, __builtin_fmaf(ca, dx, -pd.x), px[i]);
+                                py[i] = __builtin_fmaf(inv3, __builtin_fmaf(ca, dy, -pd.y), py[i]);
+                                pz[i] = __builtin_fmaf(inv3, __builtin_fmaf(ca, dz, -pd.z), pz[i]);
+                            } else {
+                                const float ca = r.q * inv3;
+                                px[i] = __builtin_fmaf(ca, dx, px[i]);
+                                py[i] = __builtin_fmaf(ca, dy, py[i]);
+                                pz[i] = __builtin_fmaf(ca, dz, pz[i]);
+                            }
+                        }
+                        if (COUNT) {
+                            const uint64_t m_chg = ballot(dip ? r.part != 0u : r.q != 0);
+                            ncell[i] += lane_of(m_use & ~m_leaf & m_chg) ? 1u : 0u;
+                            uint64_t m_far = ~0ull;  // a coincident leaf does not count
+                            if constexpr (!F64)
+                                m_far = ballot(tx[i] != r.cx || ty[i] != r.cy || tz[i] != r.cz);
+                            nleaf[i] += lane_of(m_use & m_leaf & m_far) ? 1u : 0u;
+                            nopen[i] += lane_of(m_op) ? 1u : 0u;
+                        }
+                        m_open |= m_op;
+                        if (T > 1) y |= lane_of(m_op) ? 256u << i : 0u;
                     }
                     // push the opened ranges
                     const uint64_t m_bad = m_open & ballot(r.first + r.cnt > io.n_rec);
@@ -1205,43 +1258,53 @@ __global__ __launch_bounds__(BT) void k_walk1(const InstParams* __restrict__ P, 
                     } else {
                         const uint32_t below = __builtin_amdgcn_mbcnt_hi(
                             (uint32_t)(m_open >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m_open, 0u));
-                        if (lane_of(m_open)) s_stk[base + (int)below] = make_uint2(r.first * U, r.cnt);
+                        if (lane_of(m_open)) s_stk[base + (int)below] = make_uint2(r.first * U, y);
                         sp = base + ns;
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
                 if constexpr (!F64) {
-                    kahan_add(fx, kx, px);
-                    kahan_add(fy, ky, py);
-                    kahan_add(fz, kz, pz);
+#pragma unroll
+                    for (int i = 0; i < T; i++) {
+                        kahan_add(fx[i], kx[i], px[i]);
+                        kahan_add(fy[i], ky[i], py[i]);
+                        kahan_add(fz[i], kz[i], pz[i]);
+                    }
                 }
-            }
-            if constexpr (!F64) {
-                ex = (double)fx - (double)kx;
-                ey = (double)fy - (double)ky;
-                ez = (double)fz - (double)kz;
             }
             const double K = F64 ? QE / K4PE0 : QE / (K4PE0 * p.R * p.R);
-            const double e = KIND == KIND_FIELD ? wave_sum3(ex, ey, ez) : wave_sum3(ex, 0.0, 0.0);
-            // x from lane 15, z from 31, y from 47; a potential from lane 15
-            if ((lane & 15u) == 15u && lane < (KIND == KIND_FIELD ? 48u : 16u)) {
-                double* o = io.out + (KIND == KIND_FIELD
-                                          ? 3 * (size_t)k + (lane == 15u ? 0u : (lane == 31u ? 2u : 1u))
-                                          : (size_t)k);
-                *o = (io.acc ? *o : 0.0) + K * e;
-            }
-            if (COUNT && io.counts) {
-                const uint32_t nc = wave_sum_u(ncell), nl = wave_sum_u(nleaf), no = wave_sum_u(nopen);
-                if (lane == 0) {
-                    io.counts[3 * k] = nc;
-                    io.counts[3 * k + 1] = nl;
-                    io.counts[3 * k + 2] = no;
-                }
-            }
-            tot_cell += ncell;
-            tot_leaf += nleaf;
-            tot_open += nopen;
             tot_pops += loads;
+#pragma unroll
+            for (int i = 0; i < T; i++) {
+                if (T > 1 && !((have >> i) & 1u)) continue;
+                const uint32_t k = k0 + src[i];
+                if constexpr (!F64) {
+                    ex[i] = (double)fx[i] - (double)kx[i];
+                    ey[i] = (double)fy[i] - (double)ky[i];
+                    ez[i] = (double)fz[i] - (double)kz[i];
+                }
+                const double e = KIND == KIND_FIELD ? wave_sum3(ex[i], ey[i], ez[i])
+                                                    : wave_sum3(ex[i], 0.0, 0.0);
+                // x from lane 15, z from 31, y from 47; a potential from lane 15
+                if ((lane & 15u) == 15u && lane < (KIND == KIND_FIELD ? 48u : 16u)) {
+                    double* o = io.out + (KIND == KIND_FIELD
+                                              ? 3 * (size_t)k + (lane == 15u ? 0u : (lane == 31u ? 2u : 1u))
+                                              : (size_t)k);
+                    *o = (io.acc ? *o : 0.0) + K * e;
+                }
+                if (COUNT && io.counts) {
+                    const uint32_t nc = wave_sum_u(ncell[i]), nl = wave_sum_u(nleaf[i]),
+                                   no = wave_sum_u(nopen[i]);
+                    if (lane == 0) {
+                        io.counts[3 * k] = nc;
+                        io.counts[3 * k + 1] = nl;
+                        io.counts[3 * k + 2] = no;
+                    }
+                }
+                tot_cell += ncell[i];
+                tot_leaf += nleaf[i];
+                tot_open += nopen[i];
+            }
         }
     }
     if (COUNT && KIND == KIND_FIELD) {
@@ -1281,7 +1344,7 @@ __global__ __launch_bounds__(BT) void k_walkg(const InstParams* __restrict__ P, 
                                                PState st, const NodeRec32* __restrict__ rec,
                                                WalkIO io)
 {
-    static_assert(K == 16, "group width");
+    static_assert(K == 8 || K == 16, "group width");
     constexpr uint32_t S = WAVE / K;
     constexpr uint32_t KMASK = (1u << K) - 1u;
     // a visit pops one range and pushes at most 8, so the stack holds at
@@ -1767,20 +1830,21 @@ void launch_walk_init(Bufs& b, hipStream_t s)
 // n: targets at most (step walks: half of it in most steps).  Targets per
 // wavefront: as many, up to 8, as still leave four rounds of 8 blocks per CU
 // -- a target alone keeps every wavefront of a small context busy, several
-// share the latency of reading the targets.  Walk ms at 1 / 2 / 4 / 8: 16k
-// particles 0.028 / 0.029 / 0.042 / 0.071, 150k (theta 0.8) 0.103 / 0.089 /
+// share the latency of reading the targets.  Walk ms with T = 1 at 1 / 2 / 4 / 8:
+// 16k particles 0.028 / 0.029 / 0.042 / 0.071, 150k (theta 0.8) 0.103 / 0.089 /
 // 0.088 / 0.094, 2M 2.70 / 2.57 / 2.51 / 2.47.
-template <bool F64, int MODE, int KIND, bool COUNT>
+template <int T, bool F64, int MODE, int KIND, bool COUNT>
 static void launch_walk1(Bufs& b, uint32_t n, const WalkIO& io, hipStream_t s)
 {
     const uint32_t round = NW * 8u * (uint32_t)device_cus();
-    uint32_t pw = (MODE == MODE_STEP ? n / 2 : n) / (4u * round);
-    pw = pw < 1 ? 1 : (pw > 8 ? 8 : pw);
+    const uint32_t fit = (MODE == MODE_STEP ? n / 2 : n) / (4u * round);
+    uint32_t pw = T;
+    while (pw < 8u && 2u * pw <= fit) pw *= 2u;
     uint32_t blocks = (n + NW * pw - 1) / (NW * pw);
     blocks = (blocks + XCDS - 1) / XCDS * XCDS;
     if (blocks > 65536u) blocks = 65536u;
 #define POTG_W1(DIP, REC) \
-    k_walk1<F64, MODE, KIND, DIP, COUNT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, REC, io, pw)
+    k_walk1<T, F64, MODE, KIND, DIP, COUNT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, REC, io, pw)
     if constexpr (F64) {
         if (b.dip64) POTG_W1(true, b.rec64);
         else POTG_W1(false, b.rec64);
@@ -1792,11 +1856,12 @@ static void launch_walk1(Bufs& b, uint32_t n, const WalkIO& io, hipStream_t s)
 }
 
 // float32 field walk of the chosen shape: the group criterion
-// (k_walk32grp), one target per wavefront at a time (k_walk1: group 8, and
-// point queries unless another shape was set), groups of 16 targets
-// (k_walkg), or 64 targets stepping through the children (k_walk32s, k_walk32); instantiated with dipole support only
-// for contexts holding DIPOLES instances, and with interaction counting
-// (COUNT) for point queries and for step walks while the context counts
+// (k_walk32grp); groups of 8 or 16 targets (k_walkg); 64 targets sweeping
+// whole ranges (k_walk32s: group 64, variant 1) or visiting a range's cells
+// until some open one (k_walk32).  Point queries take k_walk1 unless groups of
+// 16 or k_walk32 were set.  Instantiated with dipole support only for contexts
+// holding DIPOLES instances, and with interaction counting (COUNT) for point
+// queries and for step walks while the context counts.
 template <int MODE, bool COUNT>
 static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
 {
@@ -1805,11 +1870,14 @@ static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
     if (b.precision == POTG_MIXED_GROUP) {
         if (dip) POTG_W32((k_walk32grp<MODE, true, COUNT>));
         else POTG_W32((k_walk32grp<MODE, false, COUNT>));
-    } else if (b.group == 8 || (MODE == MODE_POINTS && b.group == 64 && b.variant == 1)) {
-        // points come in the caller's order, as often as not scattered
-        launch_walk1<false, MODE, KIND_FIELD, COUNT>(b, MODE == MODE_STEP ? b.t_cap : io.n_pts, io, s);
-    } else if (b.group == 64 && b.variant == 1) {
-        if constexpr (MODE == MODE_STEP) {
+    } else if (b.group == 8 || (b.group == 64 && b.variant == 1)) {
+        if constexpr (MODE == MODE_POINTS) {
+            // in the caller's order, as often as not scattered
+            launch_walk1<1, false, MODE, KIND_FIELD, COUNT>(b, io.n_pts, io, s);
+        } else if (b.group == 8) {
+            if (dip) POTG_W32((k_walkg<8, MODE, true, COUNT>));
+            else POTG_W32((k_walkg<8, MODE, false, COUNT>));
+        } else {
             if (dip) POTG_W32((k_walk32s<MODE, true, COUNT>));
             else POTG_W32((k_walk32s<MODE, false, COUNT>));
         }
@@ -1846,11 +1914,11 @@ static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream
 {
     const bool all = b.n_lone64 == b.n_inst;
     if (b.n_lone64) {
-        io.pick = all ? PICK_ALL : PICK_LONE | PICK_F64;
-        launch_walk1<true, MODE, KIND, COUNT>(b, n, io, s);
+        io.pick = all ? PICK_ALL : PICK_LONE;
+        launch_walk1<MODE == MODE_STEP ? 2 : 1, true, MODE, KIND, COUNT>(b, n, io, s);
     }
     if (!all) {
-        io.pick = b.n_lone64 ? PICK_SHARED | PICK_F64 : PICK_ALL;
+        io.pick = b.n_lone64 ? PICK_SHARED : PICK_ALL;
         launch_walk64c<MODE, KIND, COUNT>(b, blocks, io, s);
     }
 }
@@ -1888,7 +1956,7 @@ void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s)
     const uint32_t nb = (n + BT - 1) / BT ? (n + BT - 1) / BT : 1;
     if (kind == 1) {
         if (io.acc) k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-        launch_walk1<true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
+        launch_walk1<1, true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
         return;
     }
     if (io.acc) k_grain_init<MODE_POINTS, KIND_FIELD><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
@@ -1897,7 +1965,7 @@ void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s)
         const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
         launch_walk32<MODE_POINTS>(b, blocks, io, s);
     } else {
-        launch_walk1<true, MODE_POINTS, KIND_FIELD, true>(b, n, io, s);
+        launch_walk1<1, true, MODE_POINTS, KIND_FIELD, true>(b, n, io, s);
     }
 }
 
@@ -2069,7 +2137,7 @@ void launch_phi_noalloc(Bufs& b, uint32_t* scr, uint32_t inst, const double* pts
     const uint32_t nb = (n + BT - 1) / BT ? (n + BT - 1) / BT : 1;
     k_noalloc_prep<<<nb, BT, 0, s>>>(scr, inst, n);
     if (io.acc) k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-    launch_walk1<true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
+    launch_walk1<1, true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
 }
 
 }  // namespace potg
