@@ -410,6 +410,7 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
         c->hp[i].tree_n = (uint32_t)configs[i].N - (configs[i].geometry != POTG_SPHERE ? 1 : 0);
         c->hp[i].lone64 = lone64_rule(c->hp[i]);
         b.n_lone64 += c->hp[i].lone64 != 0;
+        b.any_bare |= c->hp[i].tree_n <= 1;
         off += (uint32_t)configs[i].N;
         tb += c->hp[i].tree_n;
     }
@@ -427,20 +428,30 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
     rc |= alloc_n(c, &b.key, n) | alloc_n(c, &b.key_alt, n);
     rc |= alloc_n(c, &b.perm, n) | alloc_n(c, &b.perm_alt, n);
     rc |= alloc_n(c, &b.sort_tmp, radix_temp_words((uint32_t)n));
-    rc |= alloc_n(c, &b.scan_tmp, scan_temp_words((uint32_t)(8 * n + 64)));
     // internal nodes: about N/2 for uniform particles (single-child chains
     // between close pairs add a few percent); 2N + 64 leaves ample room and
     // every kernel checks the bound
     const size_t ci = 2 * nt + 64;
     b.cap_int = (uint32_t)ci;
-    rc |= alloc_n(c, &b.lcp, nt) | alloc_n(c, &b.cnt, nt) | alloc_n(c, &b.base, nt);
+    rc |= alloc_n(c, &b.lcp, nt) | alloc_n(c, &b.base, nt);
+    rc |= alloc_n(c, &b.scan_tmp, scan_blocks((uint32_t)ci));
     rc |= alloc_n(c, &b.owner, ci) | alloc_n(c, &b.level, ci);
     rc |= alloc_n(c, &b.slots, 8 * ci) | alloc_n(c, &b.ccount, ci) | alloc_n(c, &b.cfirst, ci);
     rc |= alloc_n(c, &b.wid_int, ci) | alloc_n(c, &b.wid_leaf, nt);
     rc |= alloc_n(c, &b.size2, ci);
-    rc |= alloc_n(c, &b.lvl_hist, (size_t)MAXD * LVL_BLOCKS);
-    rc |= alloc_n(c, &b.lvl_off, (size_t)MAXD * LVL_BLOCKS);
-    rc |= alloc_n(c, &b.lvl_start, MAXD + 1) | alloc_n(c, &b.by_level, ci);
+    MomentLists& ml = b.ml;
+    if (b.n_tree < MOM_MAX) {
+        const uint32_t mb = moment_blocks((uint32_t)ci);
+        ml.group = mb <= MOM_ONE ? mb : MOM_GROUP;
+        ml.n_groups = (mb + ml.group - 1) / ml.group;
+        rc |= alloc_n(c, &ml.n_list, ml.n_groups) | alloc_n(c, &ml.list, (size_t)mb * MOM_LIST);
+        rc |= alloc_n(c, &ml.n_top, 1) | alloc_n(c, &ml.top, (size_t)ml.n_groups * MOM_LIST);
+        rc |= alloc_n(c, &ml.block_min, mb);
+    } else {
+        rc |= alloc_n(c, &b.lvl_hist, (size_t)MAXD * LVL_BLOCKS);
+        rc |= alloc_n(c, &b.lvl_off, (size_t)MAXD * LVL_BLOCKS);
+        rc |= alloc_n(c, &b.lvl_start, MAXD + 1) | alloc_n(c, &b.by_level, ci);
+    }
     b.n_rec = (uint32_t)(ci + nt + n_inst + 8);
     // the group walk packs a child range as first | (cnt - 1) << 29
     if (!rc && precision == POTG_MIXED_GROUP && b.n_rec >= (1u << 29)) {

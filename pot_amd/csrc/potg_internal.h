@@ -15,12 +15,44 @@ struct PState {
     uint8_t* spec;
 };
 
+// the moment pass: a block's nodes and threads (four a node), and the most
+// nodes that it can leave to the next launch, one a level
+constexpr int MOM_NODES = 256, MOM_BT = 4 * MOM_NODES;
+constexpr int MOM_LIST = MAXD + 1;
+// blocks whose lists one block of the next launch takes: all of MOM_ONE or
+// fewer, which saves a launch (a block has lanes for MOM_NODES nodes, and is
+// left some five by each)
+constexpr uint32_t MOM_GROUP = 32, MOM_ONE = 160;
+// contexts of more tree particles go up level by level, a launch each, their
+// nodes bucketed by depth: there the throughput counts, not the launches'
+// latency.  Both ways, leaf records included, us at 16k / 150k / 300k / 500k
+// / 2M particles: by level 95 / 105 / 109 / 131 / 277, here 38 / 78 / 95 /
+// 122 / 360
+constexpr uint32_t MOM_MAX = 600000;
+inline uint32_t moment_blocks(uint32_t cap) { return (cap + MOM_NODES - 1) / MOM_NODES; }
+// The moment pass' nodes that reach into the next block, by group of blocks,
+// and of these the ones that reach into the next group
+struct MomentItem {
+    uint32_t k, w, first;  // node, its record's and its first child's place
+    uint16_t cnt;
+    int16_t level;
+    uint32_t inst, pad;
+    double size2;
+};
+struct MomentLists {
+    uint32_t group, n_groups;  // group = 0: the moments are computed level by level
+    uint32_t *n_list, *n_top;  // [n_groups], [1]
+    MomentItem *list, *top;    // [blocks * MOM_LIST], [n_groups * MOM_LIST]
+    int32_t* block_min;        // lowest level of a block's nodes
+};
+
 struct Bufs {
     uint32_t n_total;  // particle slots over all instances
     uint32_t n_tree;   // leading sorted slots that belong to the trees
     uint32_t n_inst;
     int precision;     // POTG_FP64 / POTG_MIXED / POTG_MIXED_GROUP
     int any_spheroid;  // some instance has the analytic spheroid grain
+    int any_bare;      // some instance's tree has no internal nodes
     uint32_t n_lone64; // instances with lone64
     int count;         // step walks keep the interaction counters (potg_set_counting)
     int key_levels;    // digits carried by a sort key
@@ -36,10 +68,9 @@ struct Bufs {
     uint64_t *key, *key_alt;
     uint32_t *perm, *perm_alt;
     uint32_t* sort_tmp;
-    uint32_t* scan_tmp;
+    uint32_t* scan_tmp;  // tile sums of a scan
     // tree
     int32_t* lcp;
-    uint32_t* cnt;
     uint32_t* base;
     uint32_t* owner;
     int32_t* level;
@@ -51,6 +82,7 @@ struct Bufs {
     uint32_t *lvl_hist, *lvl_off;  // per-block depth histograms and their scan
     uint32_t* lvl_start;           // first slot of each depth in by_level
     uint32_t* by_level;  // internal node ids grouped by depth
+    MomentLists ml;
     double* size2;
     NodeRec64* rec64;
     NodeRec32* rec32;

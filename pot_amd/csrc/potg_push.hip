@@ -637,14 +637,72 @@ __global__ __launch_bounds__(BT) void k_reinject(const InstParams* __restrict__ 
     }
 }
 
-__global__ void k_target_flags(const InstParams* __restrict__ P, const InstState* __restrict__ S,
-                               PState st, uint32_t n_tree, uint32_t* __restrict__ flags)
+// whether tree slot i is stepped this step
+__device__ inline bool is_target(uint32_t i, const InstParams* __restrict__ P,
+                                 const InstState* __restrict__ S, const PState& st)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_tree) return;
     const uint32_t inst = st.inst[i];
-    const uint32_t local = st.ref[i] - P[inst].offset;
-    flags[i] = (st.spec[i] != 0 && local >= S[inst].start && !S[inst].retired) ? 1u : 0u;
+    return st.spec[i] != 0 && st.ref[i] - P[inst].offset >= S[inst].start && !S[inst].retired;
+}
+
+__global__ __launch_bounds__(SCAN_BT) void k_target_flags(const InstParams* __restrict__ P,
+                                                          const InstState* __restrict__ S,
+                                                          PState st, uint32_t n_tree,
+                                                          uint32_t* __restrict__ flags,
+                                                          uint32_t* __restrict__ part)
+{
+    __shared__ uint32_t sh_w[SCAN_BT / WAVE];
+    uint32_t sum = 0, total;
+#pragma unroll
+    for (int k = 0; k < SCAN_IPT; k++) {
+        const uint32_t i = blockIdx.x * SCAN_TILE + k * SCAN_BT + threadIdx.x;
+        if (i >= n_tree) continue;
+        const uint32_t f = is_target(i, P, S, st) ? 1u : 0u;
+        flags[i] = f;
+        sum += f;
+    }
+    block_excl_scan(sum, sh_w, &total);
+    if (threadIdx.x == 0) part[blockIdx.x] = total;
+}
+
+// targets before slot i, for the instances' bases; with one instance, whose
+// run starts at 0, the target list itself, its end filled up to a multiple
+// of 64 with NONE
+__global__ __launch_bounds__(SCAN_BT) void k_target_scan(const uint32_t* __restrict__ flags,
+                                                         const uint32_t* __restrict__ part,
+                                                         uint32_t n_tree, int one,
+                                                         uint32_t* __restrict__ tpos,
+                                                         uint32_t* __restrict__ targets, Globals* g)
+{
+    __shared__ uint32_t sh[SCAN_TILE];
+    __shared__ uint32_t sh_w[SCAN_BT / WAVE];
+    const uint32_t t0 = blockIdx.x * SCAN_TILE;
+    const uint32_t off = sum_before(part, blockIdx.x, sh_w);
+    uint32_t f[SCAN_IPT];
+#pragma unroll
+    for (int k = 0; k < SCAN_IPT; k++) {
+        const uint32_t j = k * SCAN_BT + threadIdx.x;
+        f[k] = t0 + j < n_tree ? flags[t0 + j] : 0u;
+        sh[j] = f[k];
+    }
+    const uint32_t total = tile_excl_scan(sh, off, sh_w);
+#pragma unroll
+    for (int k = 0; k < SCAN_IPT; k++) {
+        const uint32_t j = k * SCAN_BT + threadIdx.x;
+        if (!one) {
+            if (t0 + j < n_tree) tpos[t0 + j] = sh[j];
+        } else if (f[k]) {
+            targets[sh[j]] = t0 + j;
+        }
+    }
+    if (blockIdx.x == gridDim.x - 1) {
+        const uint32_t n = off + total, end = (n + WAVE - 1) / WAVE * WAVE;
+        if (threadIdx.x == 0) {
+            g->n_targets_real = n;
+            if (one) g->n_targets = end;
+        }
+        if (one && n + threadIdx.x < end) targets[n + threadIdx.x] = NONE;
+    }
 }
 
 // The step's targets grouped by instance, each instance's run starting at a
@@ -965,9 +1023,11 @@ __global__ __launch_bounds__(BT) void k_direct_reduce(const InstParams* __restri
 
 void launch_targets(Bufs& b, hipStream_t s)
 {
-    k_target_flags<<<grid(b.n_tree), BT, 0, s>>>(b.P, b.S, b.st, b.n_tree, b.flags);
-    exclusive_scan(b.flags, b.tpos, b.n_tree, nullptr, &b.g->n_targets_real, nullptr, b.scan_tmp,
-                   0, s);
+    const uint32_t nb = scan_blocks(b.n_tree);
+    const int one = b.n_inst == 1;
+    k_target_flags<<<nb, SCAN_BT, 0, s>>>(b.P, b.S, b.st, b.n_tree, b.flags, b.scan_tmp);
+    k_target_scan<<<nb, SCAN_BT, 0, s>>>(b.flags, b.scan_tmp, b.n_tree, one, b.tpos, b.targets, b.g);
+    if (one) return;
     k_target_bases<<<1, 1024, 0, s>>>(b.P, b.n_inst, b.n_tree, b.flags, b.tpos, b.t_first,
                                       b.t_base, b.targets, b.g);
     k_scatter_targets<<<grid(b.n_tree), BT, 0, s>>>(b.st, b.n_tree, b.flags, b.tpos, b.t_first,
