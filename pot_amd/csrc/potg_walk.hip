@@ -96,7 +96,8 @@ __device__ inline double bcast_d(double v, uint32_t j)
 // particle where the state has it (velocity Verlet / Euler-Richardson, whose
 // fields are taken at the start and the intermediate state, pot.c:2483-2485,
 // 2603-2605), or a point
-template <int MODE>
+// (PICK: only of the instances that io.pick names)
+template <int MODE, bool PICK = false>
 __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, const WalkIO& io,
                                    uint32_t k, uint32_t ntg, uint32_t& inst, uint32_t& self,
                                    double& tx, double& ty, double& tz)
@@ -110,7 +111,7 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
         if (i == NONE) return false;  // the gap before the next instance's targets
         self = i;
         inst = st.inst[i];
-        if (!picked(P[inst], io.pick)) return false;
+        if (PICK && !picked(P[inst], io.pick)) return false;
         if (P[inst].integrator == 0) {
             const double dts = P[inst].dt * (double)P[inst].tss[st.spec[i]];
             tx = st.x[i] + (0.5 * dts) * st.vx[i];
@@ -124,7 +125,7 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
     } else if (MODE == MODE_EPE) {
         self = k;
         inst = st.inst[k];
-        if (!picked(P[inst], io.pick)) return false;
+        if (PICK && !picked(P[inst], io.pick)) return false;
         const int sp = st.spec[k];
         // Boris half-drifted the stepped particles in place; the other
         // integrators' state already holds the intermediate state
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
         const uint32_t k = tile * WAVE + lane;
         uint32_t inst, self;
         double tx, ty, tz;
-        const bool valid = load_target<MODE>(P, st, io, k, ntg, inst, self, tx, ty, tz);
+        const bool valid = load_target<MODE, MODE != MODE_POINTS>(P, st, io, k, ntg, inst, self, tx, ty, tz);
         double ex = 0.0, ey = 0.0, ez = 0.0;  // the sums (ex: a potential's)
         uint32_t ncell = 0, nleaf = 0, nopen = 0;
 
@@ -1067,7 +1068,7 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
         const uint32_t k0 = (tile * NW + wv) * per_wave;
         uint32_t l_inst, l_self;
         double l_x, l_y, l_z;
-        const bool valid = load_target<MODE>(P, st, io, k0 + lane, lane < per_wave ? ntg : 0u, l_inst,
+        const bool valid = load_target<MODE, F64 && MODE != MODE_POINTS>(P, st, io, k0 + lane, lane < per_wave ? ntg : 0u, l_inst,
                                              l_self, l_x, l_y, l_z);
         float l_fx = 0.f, l_fy = 0.f, l_fz = 0.f, l_soft2 = 0.f;
         if constexpr (!F64) {
