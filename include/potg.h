@@ -165,7 +165,8 @@ typedef struct potg_tuning {
     uint32_t variant;     /* float32 walk with 64 targets: 0 visits a range's
                              cells until some lanes open one, 1 sweeps every
                              range whole before descending */
-    uint32_t sort_tile;   /* keys per tile of the radix sort: 2048 or 4096 */
+    uint32_t sort_tile;   /* keys per tile of the radix sort: 2048 or 4096
+                             (no effect below 900000 particles) */
     double walk_ms;       /* potg_tune: the chosen walk's time (ms) */
 } potg_tuning;
 

@@ -427,7 +427,7 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
     rc |= alloc_n(c, &b.P, n_inst) | alloc_n(c, &b.S, n_inst) | alloc_n(c, &b.g, 1);
     rc |= alloc_n(c, &b.key, n) | alloc_n(c, &b.key_alt, n);
     rc |= alloc_n(c, &b.perm, n) | alloc_n(c, &b.perm_alt, n);
-    rc |= alloc_n(c, &b.sort_tmp, radix_temp_words((uint32_t)n));
+    if (n >= MERGE_MAX) rc |= alloc_n(c, &b.sort_tmp, radix_temp_words((uint32_t)n));
     // internal nodes: about N/2 for uniform particles (single-child chains
     // between close pairs add a few percent); 2N + 64 leaves ample room and
     // every kernel checks the bound

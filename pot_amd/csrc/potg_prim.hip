@@ -1,4 +1,4 @@
-// potg_prim.hip -- LSD radix sort for gfx950.
+// potg_prim.hip -- sorts for gfx950.
 //
 // Written for wave64: ranks inside a wavefront come from ballots, block
 // partials through LDS.  Every routine takes an optional device-resident
@@ -181,6 +181,61 @@ __global__ __launch_bounds__(BT) void k_rs_scatter(const uint64_t* __restrict__ 
     }
 }
 
+// ---- merge sort -------------------------------------------------------
+//
+// For keys too few to fill the device: sorted tiles (sort_tile, by the kernel
+// that computes the keys), then passes that each merge a few sorted runs
+// into one.  A thread finds its element's place by a binary search in every
+// other run of its group, SEARCHES of them in flight together: a pass is bound
+// by the latency of one search (16k keys 7 us), and from some 200k keys on by
+// the searches' loads (300k 9 to 15 us, four runs to one).
+template <int SEARCHES>
+__global__ __launch_bounds__(BT) void k_merge(const uint64_t* __restrict__ kin,
+                                              const uint32_t* __restrict__ vin,
+                                              uint64_t* __restrict__ kout,
+                                              uint32_t* __restrict__ vout, uint32_t n, uint32_t len,
+                                              uint32_t len_p2, uint32_t ways)
+{
+    const uint32_t i = blockIdx.x * BT + threadIdx.x;
+    if (i >= n) return;
+    const uint64_t key = kin[i];
+    const uint32_t val = vin[i];
+    const uint32_t run = i / len, r0 = run / ways * ways;
+    const uint32_t own = run - r0, g0 = r0 * len;  // the group's first element
+    const uint32_t left = (n - g0 - 1) / len + 1;  // runs to the end, of which the last may be short
+    const uint32_t runs = left < ways ? left : ways;
+    uint32_t rank = i - run * len;
+    // elements before it: of the runs before its own those not above its
+    // key, of the runs behind those below it, so that equal keys keep their order
+    for (uint32_t q = 0; q < runs; q += SEARCHES) {
+        uint32_t pos[SEARCHES] = {}, beg[SEARCHES], m[SEARCHES];
+#pragma unroll
+        for (int k = 0; k < SEARCHES; k++) {
+            const uint32_t r = q + k;
+            beg[k] = r < runs ? g0 + r * len : i;
+            m[k] = r < runs && r != own ? (n - beg[k] < len ? n - beg[k] : len) : 0u;
+        }
+        for (uint32_t h = len_p2; h; h >>= 1) {
+            uint64_t o[SEARCHES];
+#pragma unroll
+            for (int k = 0; k < SEARCHES; k++) {
+                const uint32_t e = pos[k] + h;
+                o[k] = kin[e <= m[k] ? beg[k] + e - 1 : i];
+            }
+#pragma unroll
+            for (int k = 0; k < SEARCHES; k++) {
+                const uint32_t e = pos[k] + h;
+                const bool before = (o[k] < key) | ((o[k] == key) & (q + k < own));
+                pos[k] = (e <= m[k]) & before ? e : pos[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < SEARCHES; k++) rank += pos[k];
+    }
+    kout[g0 + rank] = key;
+    vout[g0 + rank] = val;
+}
+
 }  // namespace
 
 // sized for the smaller tile, which needs more per-tile counts
@@ -205,6 +260,24 @@ void radix_sort_pairs(uint64_t*& keys, uint64_t*& keys_alt, uint32_t*& vals, uin
                                                 tot);
         uint64_t* tk = keys; keys = keys_alt; keys_alt = tk;
         uint32_t* tv = vals; vals = vals_alt; vals_alt = tv;
+    }
+}
+
+void merge_tiles(uint64_t* keys, uint64_t* keys_alt, uint32_t* vals, uint32_t* vals_alt, uint32_t n,
+                 hipStream_t s)
+{
+    // the last pass ends in keys
+    uint32_t passes;
+    const uint32_t ways = merge_ways(n, &passes);
+    auto* merge = ways <= 4 ? k_merge<4> : (ways <= 6 ? k_merge<6> : k_merge<8>);
+    uint64_t len = MERGE_TILE;
+    for (uint32_t p = 0; p < passes; p++, len *= ways) {
+        const bool alt = (passes - p) & 1;
+        uint32_t p2 = 1;
+        while (p2 < len) p2 *= 2;
+        merge<<<(n + BT - 1) / BT, BT, 0, s>>>(alt ? keys_alt : keys, alt ? vals_alt : vals,
+                                                 alt ? keys : keys_alt, alt ? vals : vals_alt, n,
+                                                 (uint32_t)len, p2, ways);
     }
 }
 

@@ -8,8 +8,8 @@
 //   1. keys: every particle descends key_levels levels of the same
 //      recurrence; the digits (numbered in the reference's child order)
 //      form a sort key behind the instance number;
-//   2. an LSD radix sort orders the particles; runs of equal keys are
-//      ordered by descending further (rare);
+//   2. a merge sort (or an LSD radix sort, of many) orders the particles;
+//      runs of equal keys are ordered by descending further (rare);
 //   3. lcp[i] = number of leading digits particles i and i+1 share;
 //      internal node (a, l) exists for every level l with
 //      lcp[a-1] < l <= lcp[a] -- numbering the nodes by (a, l) gives a
@@ -102,38 +102,84 @@ __global__ void k_begin_step(InstParams* __restrict__ P, InstState* __restrict__
     }
 }
 
+// the low 21 bits of v, two zeros behind each
+__device__ inline uint64_t spread3(uint32_t v)
+{
+    uint64_t x = v & 0x1fffffu;
+    x = (x | x << 32) & 0x001f00000000ffffull;
+    x = (x | x << 16) & 0x001f0000ff0000ffull;
+    x = (x | x << 8) & 0x100f00f00f00f00full;
+    x = (x | x << 4) & 0x10c30c30c30c30c3ull;
+    return (x | x << 2) & 0x1249249249249249ull;
+}
+
+// the key of the particle in slot i
+__device__ inline uint64_t key_of(uint32_t i, const InstParams* __restrict__ P, const PState& st,
+                                  int levels, Globals* g)
+{
+    const uint32_t inst = st.inst[i];
+    const InstParams& p = P[inst];
+    // the analytic spheroid grain stays out of the tree (SPH:1516-1521)
+    if (p.geometry != 0 && st.spec[i] == 0) return ~0ull;
+    const double px = st.x[i], py = st.y[i], pz = st.z[i];
+    const double r2 = p.root_x2;
+    if (!(px >= 0.0) || px > r2 || !(py >= 0.0) || py > r2 || !(pz >= 0.0) || pz > r2) {
+        raise_err(g, KERR_OUT_OF_BOX, st.ref[i]);
+        return (uint64_t)inst << (3 * levels);
+    }
+    // The position in cells of the last level (at most 2^21 along a side).
+    // It carries an error below 2^-30 cells and the recurrence's midpoints
+    // one below 2^-27, so further than 2^-20 from a face its whole part holds
+    // the recurrence's decisions.  (The recurrence for every particle, 440
+    // float64 instructions: 2M keys 38 us instead of 22.)
+    const double scale = p.invR * (double)(1u << (levels - 1));
+    const double cx = px * scale, cy = py * scale, cz = pz * scale;
+    const uint32_t ix = (uint32_t)cx, iy = (uint32_t)cy, iz = (uint32_t)cz;
+    const double fx = cx - (double)ix, fy = cy - (double)iy, fz = cz - (double)iz;
+    const double lo = fmin(fx, fmin(fy, fz)), hi = fmax(fx, fmax(fy, fz));
+    if (lo > 0x1p-20 && hi < 1.0 - 0x1p-20)
+        // ref_digit of every level: y, whether x and y agree, z
+        return (uint64_t)inst << (3 * levels) | spread3(iy) << 2 |
+               spread3(~(ix ^ iy) & ((1u << levels) - 1u)) << 1 | spread3(iz);
+    double x1 = 0.0, x2 = r2, y1 = 0.0, y2 = r2, z1 = 0.0, z2 = r2;
+    uint64_t k = inst;
+    for (int l = 0; l < levels; l++) k = (k << 3) | (uint64_t)descend1(px, py, pz, x1, x2, y1, y2, z1, z2);
+    return k;
+}
+
 __global__ void k_keys(const InstParams* __restrict__ P, PState st, uint32_t n, int levels,
                        uint64_t* __restrict__ key, uint32_t* __restrict__ perm, Globals* g)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     perm[i] = i;
-    const uint32_t inst = st.inst[i];
-    const InstParams& p = P[inst];
-    if (p.geometry != 0 && st.spec[i] == 0) {
-        key[i] = ~0ull;  // the analytic spheroid grain stays out of the tree (SPH:1516-1521)
-        return;
-    }
-    const double px = st.x[i], py = st.y[i], pz = st.z[i];
-    const double r2 = p.root_x2;
-    if (!(px >= 0.0) || px > r2 || !(py >= 0.0) || py > r2 || !(pz >= 0.0) || pz > r2) {
-        raise_err(g, KERR_OUT_OF_BOX, st.ref[i]);
-        key[i] = (uint64_t)inst << (3 * levels);
-        return;
-    }
-    double x1 = 0.0, x2 = r2, y1 = 0.0, y2 = r2, z1 = 0.0, z2 = r2;
-    uint64_t k = inst;
-    for (int l = 0; l < levels; l++) k = (k << 3) | (uint64_t)descend1(px, py, pz, x1, x2, y1, y2, z1, z2);
-    key[i] = k;
+    key[i] = key_of(i, P, st, levels, g);
 }
 
-// order runs of equal keys by their deeper digits (insertion sort per run)
-__global__ void k_tiefix(const uint64_t* __restrict__ key, uint32_t* __restrict__ perm,
-                         const InstParams* __restrict__ P, PState st, uint32_t n_tree, Globals* g)
+// the keys in sorted tiles
+__global__ __launch_bounds__(MERGE_TILE) void k_key_tiles(const InstParams* __restrict__ P, PState st,
+                                                          uint32_t n, int levels,
+                                                          uint64_t* __restrict__ key,
+                                                          uint32_t* __restrict__ perm, Globals* g)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i + 1 >= n_tree) return;
-    if (key[i] != key[i + 1] || (i > 0 && key[i - 1] == key[i])) return;
+    __shared__ TileSort sh;
+    const uint32_t t0 = blockIdx.x * MERGE_TILE, i = t0 + threadIdx.x;
+    // what fills the last tile sorts behind all
+    uint64_t k = i < n ? key_of(i, P, st, levels, g) : ~0ull;
+    uint32_t idx;
+    sort_tile(sh, k, idx);
+    if (i < n) {
+        key[i] = k;
+        perm[i] = t0 + idx;
+    }
+}
+
+// orders the run of equal keys from slot i by their deeper digits (insertion
+// sort); returns its end
+__device__ inline uint32_t order_ties(uint32_t i, const uint64_t* __restrict__ key, uint32_t* perm,
+                                      const InstParams* __restrict__ P, const PState& st,
+                                      uint32_t n_tree, Globals* g)
+{
     uint32_t e = i + 1;
     while (e + 1 < n_tree && key[e + 1] == key[i]) e++;
     const double r2 = P[st.inst[perm[i]]].root_x2;
@@ -146,7 +192,7 @@ __global__ void k_tiefix(const uint64_t* __restrict__ key, uint32_t* __restrict_
             const int d = split_depth(st.x[pa], st.y[pa], st.z[pa], st.x[pb], st.y[pb], st.z[pb], r2);
             if (d >= MAXD) {
                 raise_err(g, KERR_COINCIDENT, st.ref[pa]);
-                return;
+                return e + 1;
             }
             double x1, x2;
             const int da = descend_to(st.x[pa], st.y[pa], st.z[pa], r2, d + 1, x1, x2);
@@ -157,29 +203,40 @@ __global__ void k_tiefix(const uint64_t* __restrict__ key, uint32_t* __restrict_
         }
         perm[b] = pa;
     }
+    return e + 1;
 }
 
-// the particles into sorted order; the grain of each instance notes its
-// slot (the potential-energy pass reads the grain's potential there)
-__global__ void k_permute(const uint32_t* __restrict__ perm, PState src, PState dst, uint32_t n,
-                          const InstParams* __restrict__ P, InstState* __restrict__ S)
+// the particles into sorted order, runs of equal keys (rare) by the thread
+// that has the first of them; the grain of each instance notes its slot (the
+// potential-energy pass reads the grain's potential there)
+__global__ void k_permute(const uint64_t* __restrict__ key, uint32_t* perm, PState src, PState dst,
+                          uint32_t n, uint32_t n_tree, const InstParams* __restrict__ P,
+                          InstState* __restrict__ S, Globals* g)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const uint32_t j = perm[i];
-    dst.x[i] = src.x[j];
-    dst.y[i] = src.y[j];
-    dst.z[i] = src.z[j];
-    dst.vx[i] = src.vx[j];
-    dst.vy[i] = src.vy[j];
-    dst.vz[i] = src.vz[j];
-    const uint32_t r = src.ref[j];
-    const uint16_t inst = src.inst[j];
-    const uint8_t spec = src.spec[j];
-    dst.ref[i] = r;
-    dst.inst[i] = inst;
-    dst.spec[i] = spec;
-    if (spec == 0 && r == P[inst].offset) S[inst].grain_slot = i;
+    uint32_t end = i + 1;
+    if (i < n_tree) {
+        const uint64_t k = key[i];
+        if (i > 0 && key[i - 1] == k) return;
+        if (end < n_tree && key[end] == k) end = order_ties(i, key, perm, P, src, n_tree, g);
+    }
+    for (; i < end; i++) {
+        const uint32_t j = perm[i];
+        dst.x[i] = src.x[j];
+        dst.y[i] = src.y[j];
+        dst.z[i] = src.z[j];
+        dst.vx[i] = src.vx[j];
+        dst.vy[i] = src.vy[j];
+        dst.vz[i] = src.vz[j];
+        const uint32_t r = src.ref[j];
+        const uint16_t inst = src.inst[j];
+        const uint8_t spec = src.spec[j];
+        dst.ref[i] = r;
+        dst.inst[i] = inst;
+        dst.spec[i] = spec;
+        if (spec == 0 && r == P[inst].offset) S[inst].grain_slot = i;
+    }
 }
 
 // lcp[i] and the tile's count of internal nodes: particle i owns a node for
@@ -1246,11 +1303,18 @@ void launch_leaf_refresh(Bufs& b, hipStream_t s)
 
 void launch_keys_sort_permute(Bufs& b, hipStream_t s)
 {
-    k_keys<<<grid(b.n_total), BT, 0, s>>>(b.P, b.st, b.n_total, b.key_levels, b.key, b.perm, b.g);
-    radix_sort_pairs(b.key, b.key_alt, b.perm, b.perm_alt, b.n_total, b.key_bits, b.sort_tmp,
-                     (int)b.sort_ipt, s);
-    k_tiefix<<<grid(b.n_tree), BT, 0, s>>>(b.key, b.perm, b.P, b.st, b.n_tree, b.g);
-    k_permute<<<grid(b.n_total), BT, 0, s>>>(b.perm, b.st, b.alt, b.n_total, b.P, b.S);
+    const uint32_t n = b.n_total;
+    if (n < MERGE_MAX) {
+        const bool alt = merge_passes(n) & 1;
+        k_key_tiles<<<(n + MERGE_TILE - 1) / MERGE_TILE, MERGE_TILE, 0, s>>>(
+            b.P, b.st, n, b.key_levels, alt ? b.key_alt : b.key, alt ? b.perm_alt : b.perm, b.g);
+        merge_tiles(b.key, b.key_alt, b.perm, b.perm_alt, n, s);
+    } else {
+        k_keys<<<grid(n), BT, 0, s>>>(b.P, b.st, n, b.key_levels, b.key, b.perm, b.g);
+        radix_sort_pairs(b.key, b.key_alt, b.perm, b.perm_alt, n, b.key_bits, b.sort_tmp,
+                         (int)b.sort_ipt, s);
+    }
+    k_permute<<<grid(n), BT, 0, s>>>(b.key, b.perm, b.st, b.alt, n, b.n_tree, b.P, b.S, b.g);
     PState t = b.st;
     b.st = b.alt;
     b.alt = t;
