@@ -29,7 +29,7 @@ constexpr int EPE_BLOCKS = 64;    // partial sums per instance of the PE reducti
 // depths given a launch per level (the others are done by one block)
 constexpr uint32_t LVL_BLOCKS = 256;
 constexpr int LVL_WIDE_LO = 12;   // depths >= this: one block
-constexpr int LVL_WIDE_HI = 3;    // depths <= this: one block
+constexpr int LVL_WIDE_HI = 3;    // depths <= this: one block, while few nodes
 
 // error codes raised by kernels (mirrors POTG_ERR_*)
 constexpr int KERR_OUT_OF_BOX = 1;

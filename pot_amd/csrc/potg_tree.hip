@@ -1348,16 +1348,20 @@ void launch_tree(Bufs& b, hipStream_t s)
         k_level_scatter<<<LVL_BLOCKS, BT, 0, s>>>(b.level, b.g, cap, b.lvl_off, b.by_level);
         // deepest level first.  Levels below LVL_WIDE_LO hold few nodes in
         // any plasma (their cells are a few mean spacings wide or less), as
-        // do those above LVL_WIDE_HI: one block each; the levels between
-        // get a launch of their own
+        // do the top ones, at most 8^L n_inst: one block each; the levels
+        // between get a launch of their own.  (16 trees' four top levels in
+        // one block took 177 us, three and a launch 40.)
+        int hi = LVL_WIDE_HI;
+        while (hi >= 0 && ((uint64_t)b.n_inst << (3 * hi)) > 1024u) hi--;
         k_level_moments_block<<<1, 1024, 0, s>>>(MAXD - 1, LVL_WIDE_LO, b.st, b.P, b.g, cap, b.owner,
                                                  b.ccount, b.cfirst, b.wid_int, b.size2, b.rec64, r32,
                                                  b.dip64, d32, b.n_rec, b.lvl_start, b.by_level);
-        for (int L = LVL_WIDE_LO - 1; L > LVL_WIDE_HI; L--)
+        for (int L = LVL_WIDE_LO - 1; L > hi; L--)
             k_level_moments<<<gb, BT, 0, s>>>(L, b.st, b.P, b.g, cap, b.owner, b.ccount, b.cfirst,
                                               b.wid_int, b.size2, b.rec64, r32, b.dip64, d32, b.n_rec,
                                               b.lvl_start, b.by_level);
-        k_level_moments_block<<<1, 1024, 0, s>>>(LVL_WIDE_HI, 0, b.st, b.P, b.g, cap, b.owner,
+        if (hi < 0) return;
+        k_level_moments_block<<<1, 1024, 0, s>>>(hi, 0, b.st, b.P, b.g, cap, b.owner,
                                                  b.ccount, b.cfirst, b.wid_int, b.size2, b.rec64, r32,
                                                  b.dip64, d32, b.n_rec, b.lvl_start, b.by_level);
         return;

@@ -82,3 +82,20 @@ def test_batch_of_bare_trees():
         sim.build_tree()
         ref, got = sim.tree_canon(), ctx.tree_canon(k)
         _equal(got, ref)
+
+
+@pytest.mark.parametrize("n_inst,N", [(16, 37600), (40, 15100), (1100, 550)])
+def test_large_batches(n_inst, N):
+    # more tree particles than the blocks of nodes take: level by level, the
+    # top levels' nodes shared out by the number of trees
+    case = big_case(N, seed=n_inst)
+    sim = oracle_sim(case)
+    parts = sim.particles().view(G.PARTICLE_DT)
+    sim.build_tree()
+    ref = sim.tree_canon()
+    ctx = G.Context([gpu_config(case)] * n_inst, G.POTG_FP64)
+    for k in range(n_inst):
+        ctx.upload(k, parts)
+    ctx.build_tree()
+    for k in (0, 1, n_inst // 2, n_inst - 1):
+        _equal(ctx.tree_canon(k), ref)
