@@ -74,7 +74,7 @@ struct Stream {
 };
 
 // ---- SCEPTIC reinjection samplers (prng.c:138-214, pot.c:433-492) ----
-__device__ double u_no_flow_icdf(double chi, double q)
+__device__ __noinline__ double u_no_flow_icdf(double chi, double q)
 {
     const double omc = 1.0 - chi;
     double p, u = 1.29951, usq;
@@ -87,7 +87,7 @@ __device__ double u_no_flow_icdf(double chi, double q)
     return u;
 }
 
-__device__ double u_icdf(double U, double chi, double q)
+__device__ __noinline__ double u_icdf(double U, double chi, double q)
 {
     const double Usq = U * U;
     const double psi = SQRT_PI * (1.0 + (2.0 * (Usq - chi))) / 2.0;
@@ -124,19 +124,23 @@ __device__ inline double readlane_d(double v, int j)
 // with the same arguments and the same result.  The serial loop bisects a
 // panel [xi0, xi2] until the integrand is linear within max_lin_dev at its
 // midpoint: level l's midpoint is the previous level's halved towards xi0,
-// and its test reads the integrand there and at the previous level.  Here
-// lanes 0..IFA_LV-1 evaluate IFA_LV consecutive levels at once and the
-// first level that passes is the panel; the midpoints, the integrand, the
-// tests and the sum are the serial loop's float64 operations in its order,
-// so the result is the serial one bit for bit.  The serial loop's guard of
-// 4000000 bisections in all is kept.
+// and its test reads the integrand there and at the previous level.  Where a
+// panel ends, at the top of the level that passes, the next one starts.  Here
+// a lane stands for one choice of the levels that end two panels in a row
+// (IFA_LV levels each) and evaluates the two midpoints, which do not depend
+// on the integrand; the tests then pick the choice.  A panel that none of the
+// levels ends is bisected on, IFA_LV levels at once.  The midpoints, the
+// integrand, the tests and the sum are the serial loop's float64 operations
+// in its order, so the result is the serial one bit for bit.  The serial
+// loop's guard of 4000000 bisections in all is kept.  (k_reinject lasts as
+// long as its longest integral, up to some 100 panels: one panel at a time 37
+// us at 16k particles and 110 at 2M, two 28 and 86.)
 constexpr int IFA_LV = 8;  // panels deeper than 7 levels are rare
 
-__device__ double integrate_for_alpha(double s, double chi_b, double u2, double Rol,
+__device__ __noinline__ double integrate_for_alpha(double s, double chi_b, double u2, double Rol,
                                       double max_lin_dev)
 {
     const int lane = (int)__lane_id();
-    const int kl = lane < IFA_LV ? lane : IFA_LV - 1;
     const double chu2 = chi_b / u2;
     const double s2 = s * s;
     const double y_one = s / sqrt(1.0 - chu2 - s2);
@@ -145,20 +149,72 @@ __device__ double integrate_for_alpha(double s, double chi_b, double u2, double 
     double y0 = s, y1, y2;
     long guard = 0;
     if (s == 0.0) return 0.0;
-    do {
-        // levels base .. base + IFA_LV - 1 below the panel top (top, ytop)
+    const auto integrand = [&](double xi) {
+        const double y = 1.0 - (chu2 * xi * exp(Rol * (1.0 - (1.0 / xi))));
+        return 1.0 / sqrt((y / s2) - (xi * xi));
+    };
+    // the midpoint of a panel's level k and its top
+    const auto bisect = [](double from, int k, double& top) {
+        double mid = 1.0;
+        for (int j = 0; j < IFA_LV; j++) {
+            top = j <= k ? mid : top;
+            mid = j <= k ? (from + mid) / 2.0 : mid;
+        }
+        return mid;
+    };
+    const auto linear = [&](double ya, double y, double yb) {
+        return !(fabs(ya - y - (y - yb)) > max_lin_dev);
+    };
+    const int k1 = lane / IFA_LV, k2 = lane % IFA_LV;
+    for (;;) {
+        // the lane's two panels, from their tops
+        double t1 = 1.0, t2 = 1.0;
+        const double m1 = bisect(xi0, k1, t1), m2 = bisect(t1, k2, t2);
+        const double f1 = integrand(m1), f2 = integrand(m2);
+        const double g1 = __shfl(f1, (lane - IFA_LV) & 63, WAVE);
+        const double g2 = __shfl(f2, (lane - 1) & 63, WAVE);
+        const double a1 = k1 ? g1 : y_one, a2 = k2 ? g2 : y_one;
+        const uint64_t ok1 = ballot(linear(a1, f1, y0) && k2 == 0);
+        const uint64_t ok2 = ballot(linear(a2, f2, a1));
+        // the levels that end the panels: the first of the eight that passes
+        int at = 0;
+        bool deep = false, done = false;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const uint64_t ok = q == 0 ? ok1 : (ok2 >> at) & 0xffull;
+            if (!ok) {
+                deep = true;
+                break;
+            }
+            const int step = __ffsll((unsigned long long)ok) - 1;
+            at += step;
+            guard += q == 0 ? step / IFA_LV : step;
+            if (guard > 4000000) return __builtin_nan("");
+            xi2 = readlane_d(q == 0 ? t1 : t2, at);
+            y2 = readlane_d(q == 0 ? a1 : a2, at);
+            y1 = readlane_d(q == 0 ? f1 : f2, at);
+            alpha += (xi2 - xi0) * (y0 + (4.0 * y1) + y2) / 6.0;
+            xi0 = xi2;
+            y0 = y2;
+            if (!(xi2 < 1.0)) {
+                done = true;
+                break;
+            }
+        }
+        if (done) return alpha;
+        if (!deep) continue;
+        // one panel, levels base .. base + IFA_LV - 1 below its top (top, ytop)
+        const int kl = lane < IFA_LV ? lane : IFA_LV - 1;
         double top = 1.0, ytop = y_one;
         for (long base = 0;; base += IFA_LV) {
             double xi1 = top;
             for (int j = 0; j <= kl; j++) xi1 = (xi0 + xi1) / 2.0;
-            double y = 1.0 - (chu2 * xi1 * exp(Rol * (1.0 - (1.0 / xi1))));
-            y = 1.0 / sqrt((y / s2) - (xi1 * xi1));
+            const double y = integrand(xi1);
             const double xu = __shfl(xi1, lane > 0 ? lane - 1 : 0, WAVE);
             const double yu = __shfl(y, lane > 0 ? lane - 1 : 0, WAVE);
             const double xa = lane == 0 ? top : xu;   // the level above
             const double ya = lane == 0 ? ytop : yu;
-            const uint64_t pass =
-                ballot(lane < IFA_LV && !(fabs(ya - y - (y - y0)) > max_lin_dev));
+            const uint64_t pass = ballot(lane < IFA_LV && linear(ya, y, y0));
             if (pass) {
                 const int k = __ffsll((unsigned long long)pass) - 1;
                 // level base + k took base + k bisections
@@ -176,8 +232,8 @@ __device__ double integrate_for_alpha(double s, double chi_b, double u2, double 
         alpha += (xi2 - xi0) * (y0 + (4.0 * y1) + y2) / 6.0;
         xi0 = xi2;
         y0 = y2;
-    } while (xi2 < 1.0);
-    return alpha;
+        if (!(xi2 < 1.0)) return alpha;
+    }
 }
 
 // coord.c:21-35
@@ -221,6 +277,13 @@ __device__ inline void vel_cart(const double* v, double phi, double theta, doubl
     vz = (v[0] * cos(theta)) - (v[2] * sin(theta));
 }
 
+// kept out of line, as the root finders and the integral are: all inlined,
+// their constants spilled 769 scalar registers (k_reinject of 16k particles
+// 28 us, 24 out of line; of 2M 86 and 68)
+__device__ __noinline__ double sin_of(double x) { return sin(x); }
+__device__ __noinline__ double cos_of(double x) { return cos(x); }
+__device__ __noinline__ double acos_of(double x) { return acos(x); }
+
 // sceptically_reinject, pot.c:496-652.  The reference retries by recursion
 // while alpha comes out NaN (pot.c:583-598), restoring chi_b as it does; here
 // the retry is bounded.  When every try fails -- a chi_b that bars the
@@ -230,8 +293,8 @@ __device__ inline void vel_cart(const double* v, double phi, double theta, doubl
 __device__ bool sceptic_reinject(const InstParams& p, int species, double chi_b_in, Stream& rs,
                                  double& x, double& y, double& z, double& vx, double& vy, double& vz)
 {
-    double a[2], alpha = 0.0, b = 0.0, c, co_z, phi, psi, q, U, u_mag = 1.0, u2 = 1.0, v_n = 0.0;
-    double u[3] = {0.0, 0.0, 1.0}, v[3];
+    double a[2], alpha = 0.0, b = 0.0, c = 0.0, co_z, phi, psi = 0.0, q, U, u_mag = 1.0, u2 = 1.0;
+    double v_n = 0.0, u[3], v[3];
     double chi_b = chi_b_in;
     for (int tries = 0; tries < 1000; tries++) {
         v_n = 2.0 * KB / p.mass[species];
@@ -260,16 +323,7 @@ __device__ bool sceptic_reinject(const InstParams& p, int species, double chi_b_
             } while (u2 < chi_b && ++it < 100000);
             c = rs.draw(2.0) - 1.0;
         }
-        u[0] = 0.0;
-        u[1] = 0.0;
-        u[2] = u_mag;
-        a[0] = 0.0;
-        a[1] = 1.0;
-        rot_xy(a, c, sqrt(1.0 - (c * c)), u[0], u[1], u[2], 0.0);
-        a[0] = 1.0;
-        a[1] = 0.0;
         psi = rs.draw(2.0 * PI);
-        rot_xy(a, sin(psi), cos(psi), u[0], u[1], u[2], 0.0);
         b = sqrt(rs.draw(1.0 - (chi_b / u2)));
         alpha = integrate_for_alpha(b, chi_b, u2, p.Rol, p.max_lin_dev);
         if (!isnan(alpha)) break;
@@ -277,20 +331,41 @@ __device__ bool sceptic_reinject(const InstParams& p, int species, double chi_b_
     }
     if (isnan(alpha)) return false;
     phi = rs.draw(2.0 * PI);
-    x = p.R * sin(alpha) * cos(phi);
-    y = p.R * sin(alpha) * sin(phi);
-    z = p.R * cos(alpha);
+    // the three angles' sines and cosines, an angle a lane: one evaluation
+    // for the wavefront
+    const int lane = (int)__lane_id();
+    const double angle = lane == 0 ? psi : (lane == 1 ? alpha : phi);
+    const double si = sin_of(angle), co = cos_of(angle);
+    const double s_psi = readlane_d(si, 0), c_psi = readlane_d(co, 0);
+    const double s_al = readlane_d(si, 1), c_al = readlane_d(co, 1);
+    const double s_phi = readlane_d(si, 2), c_phi = readlane_d(co, 2);
+    u[0] = 0.0;
+    u[1] = 0.0;
+    u[2] = u_mag;
+    a[0] = 0.0;
+    a[1] = 1.0;
+    rot_xy(a, c, sqrt(1.0 - (c * c)), u[0], u[1], u[2], 0.0);
+    a[0] = 1.0;
+    a[1] = 0.0;
+    rot_xy(a, s_psi, c_psi, u[0], u[1], u[2], 0.0);
+    x = p.R * s_al * c_phi;
+    y = p.R * s_al * s_phi;
+    z = p.R * c_al;
     a[0] = u[1];
     a[1] = -u[0];
     a[0] /= sqrt((u[0] * u[0]) + (u[1] * u[1]));
     a[1] /= sqrt((u[0] * u[0]) + (u[1] * u[1]));
     co_z = u[2] / u_mag;
-    rot_xy(a, sin(acos(co_z)), co_z, x, y, z, p.R);
+    const double si_z = sin_of(acos_of(co_z));
+    rot_xy(a, si_z, co_z, x, y, z, p.R);
     v[1] = 0.0;
     v[2] = u_mag * b;
     v[0] = -sqrt(u2 - chi_b - (v[2] * v[2]));
-    vel_cart(v, phi, alpha, vx, vy, vz);
-    rot_xy(a, sin(acos(co_z)), co_z, vx, vy, vz, 0.0);
+    // vel_cart (coord.c:6-14) of (v, phi, alpha)
+    vx = (v[0] * c_phi * s_al) - (v[1] * s_phi) + (v[2] * c_phi * c_al);
+    vy = (v[0] * s_phi * s_al) + (v[1] * c_phi) + (v[2] * s_phi * c_al);
+    vz = (v[0] * c_al) - (v[2] * s_al);
+    rot_xy(a, si_z, co_z, vx, vy, vz, 0.0);
     vx *= v_n;
     vy *= v_n;
     vz *= v_n;
@@ -298,7 +373,7 @@ __device__ bool sceptic_reinject(const InstParams& p, int species, double chi_b_
 }
 
 // plain spherical reinjection at the boundary (inject, pot.c:710-765)
-__device__ void plain_reinject(const InstParams& p, int species, Stream& rs, double& x, double& y,
+__device__ __noinline__ void plain_reinject(const InstParams& p, int species, Stream& rs, double& x, double& y,
                                double& z, double& vx, double& vy, double& vz)
 {
     const double sigma = species == 1 ? sqrt(KB * p.Ti / p.mass[1]) : sqrt(KB * p.Te / p.mass[2]);
@@ -385,6 +460,14 @@ __device__ int bounce_off_wall(const InstParams& p, double& x, double& y, double
         z = pz;
     }
     return 0;
+}
+
+// the same out of line, for k_reinject
+__device__ __noinline__ int bounce_reinjected(const InstParams& p, double& x, double& y, double& z,
+                                              double& vx, double& vy, double& vz, double px, double py,
+                                              double pz)
+{
+    return bounce_off_wall(p, x, y, z, vx, vy, vz, px, py, pz);
 }
 
 // Velocity Verlet and Euler-Richardson, first half (pot.c:2532-2554): the
@@ -586,24 +669,27 @@ __global__ __launch_bounds__(BT) void k_reinject(const InstParams* __restrict__ 
         const double chi_b = S[inst].chi_b;
         double x = st.x[i], y = st.y[i], z = st.z[i];
         double vx = st.vx[i], vy = st.vy[i], vz = st.vz[i];
+        // an absorbed particle that lands outside the boundary is sampled a
+        // second time; the sampling stands in one place, as it fills the
+        // registers by itself
         bool ok = true;
-        if (p.sceptic) ok = sceptic_reinject(p, s, chi_b, rs, x, y, z, vx, vy, vz);
-        else plain_reinject(p, s, rs, x, y, z, vx, vy, vz);
-        if ((code & 1u) && p.out_bounce) {
-            // the absorbed particle's start position is where a bounce
-            // returns it (pot.c:2686-2690)
-            if (bounce_off_wall(p, x, y, z, vx, vy, vz, qprev[3 * (size_t)e],
-                                qprev[3 * (size_t)e + 1], qprev[3 * (size_t)e + 2]) < 0 &&
-                lane == 0)
-                atomicAdd(&S[inst].n_wall_inward, 1u);
-        } else if (code & 1u) {
+        for (int again = 0;; again++) {
+            if (p.sceptic) ok = sceptic_reinject(p, s, chi_b, rs, x, y, z, vx, vy, vz);
+            else plain_reinject(p, s, rs, x, y, z, vx, vy, vz);
+            if (again || !(code & 1u)) break;
+            if (p.out_bounce) {
+                // the absorbed particle's start position is where a bounce
+                // returns it (pot.c:2686-2690)
+                if (bounce_reinjected(p, x, y, z, vx, vy, vz, qprev[3 * (size_t)e],
+                                      qprev[3 * (size_t)e + 1], qprev[3 * (size_t)e + 2]) < 0 &&
+                    lane == 0)
+                    atomicAdd(&S[inst].n_wall_inward, 1u);
+                break;
+            }
             const double rad = p.R;
             const double dx = x - rad, dy = y - rad, dz = z - rad;
-            if (ok && sqrt(dx * dx + dy * dy + dz * dz) > rad) {
-                if (lane == 0) atomicAdd(&S[inst].n_reinj_out, 1u);
-                if (p.sceptic) ok = sceptic_reinject(p, s, chi_b, rs, x, y, z, vx, vy, vz);
-                else plain_reinject(p, s, rs, x, y, z, vx, vy, vz);
-            }
+            if (!ok || !(sqrt(dx * dx + dy * dy + dz * dz) > rad)) break;
+            if (lane == 0) atomicAdd(&S[inst].n_reinj_out, 1u);
         }
         if (!ok && !g->retire) {
             if (lane == 0) raise_err(g, KERR_REINJECT, st.ref[i]);
@@ -1038,7 +1124,7 @@ void launch_push(Bufs& b, hipStream_t s)
 {
     k_push<<<grid(b.t_cap), BT, 0, s>>>(b.P, b.S, b.g, b.st, b.targets, b.E, b.a1, b.x0, b.queue,
                                         b.qprev, b.n_tree);
-    k_reinject<<<256, BT, 0, s>>>(b.P, b.S, b.g, b.st, b.queue, b.qprev, b.n_tree);
+    k_reinject<<<1024, BT, 0, s>>>(b.P, b.S, b.g, b.st, b.queue, b.qprev, b.n_tree);
 }
 
 void launch_half(Bufs& b, hipStream_t s)
