@@ -141,8 +141,12 @@ void launch_leaf_refresh(Bufs& b, hipStream_t s);
 void launch_finish_step(Bufs& b, int compute_epe, hipStream_t s);
 void launch_epe(Bufs& b, hipStream_t s);
 // upload / download helpers
-void launch_scatter_upload(Bufs& b, uint32_t inst, const double* aos, uint32_t n, hipStream_t s);
-void launch_gather_download(Bufs& b, uint32_t inst, double* aos, uint32_t n, hipStream_t s);
+// offset: of the instance's particles in reference order.  A download puts the
+// instance's state behind its particles.
+void launch_scatter_upload(Bufs& b, uint32_t inst, uint32_t offset, const double* aos, uint32_t n,
+                           hipStream_t s);
+void launch_gather_download(Bufs& b, uint32_t inst, uint32_t offset, double* aos, uint32_t n,
+                            hipStream_t s);
 void launch_build_inverse(Bufs& b, hipStream_t s);
 // set every slot to its reference identity (at creation)
 void launch_init_slots(Bufs& b, hipStream_t s);
