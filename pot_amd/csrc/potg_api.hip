@@ -864,27 +864,15 @@ static int run_points(potg_ctx* c, uint32_t inst, const double* xyz, const uint3
                       size_t n, int kind, double* out, uint32_t* counts)
 {
     Bufs& b = c->b;
-    std::vector<uint32_t> vi, vs;
-    std::vector<uint32_t> inv(b.n_total);
-    if (kind == 0 && exclude) {
-        launch_build_inverse(b, c->stream);
-        HIPCHK(hipMemcpyAsync(inv.data(), b.inv, inv.size() * sizeof(uint32_t),
-                              hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-    }
-    const uint32_t off = c->hp[inst].offset;
+    const bool excl = kind == 0 && exclude;
+    if (excl) launch_build_inverse(b, c->stream);
+    const InstParams& p = c->hp[inst];
     for (size_t s0 = 0; s0 < n; s0 += b.q_cap) {
         const uint32_t m = (uint32_t)((n - s0) < b.q_cap ? (n - s0) : b.q_cap);
-        vi.assign(m, inst);
-        vs.assign(m, NONE);
-        if (kind == 0 && exclude)
-            for (uint32_t k = 0; k < m; k++) {
-                const uint32_t e = exclude[s0 + k];
-                vs[k] = (e == 0xFFFFFFFFu || e >= c->cfg[inst].N) ? NONE : inv[off + e];
-            }
         HIPCHK(hipMemcpyAsync(b.q_pts, xyz + 3 * s0, 3 * sizeof(double) * m, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(b.q_inst, vi.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(b.q_self, vs.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
+        if (excl)
+            HIPCHK(hipMemcpyAsync(b.q_self, exclude + s0, sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
+        launch_point_targets(b, inst, p.offset, p.N, m, excl, c->stream);
         launch_points(b, m, kind, c->stream);
         const size_t per = kind == 0 ? 3 : 1;
         HIPCHK(hipMemcpyAsync(out + per * s0, b.q_out, per * sizeof(double) * m, hipMemcpyDeviceToHost, c->stream));
@@ -975,20 +963,14 @@ int potg_direct_sum(potg_ctx* c, uint32_t inst, const uint32_t* idx, size_t n, d
     if (!c || inst >= c->b.n_inst || (n && (!idx || !E)))
         return set_err("potg_direct_sum: bad arguments"), POTG_ERR_ARG;
     Bufs& b = c->b;
-    std::vector<uint32_t> inv(b.n_total), vs;
     launch_build_inverse(b, c->stream);
-    HIPCHK(hipMemcpyAsync(inv.data(), b.inv, inv.size() * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                          c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const uint32_t off = c->hp[inst].offset;
+    const InstParams& p = c->hp[inst];
     for (size_t s0 = 0; s0 < n; s0 += b.q_cap) {
         const uint32_t m = (uint32_t)((n - s0) < b.q_cap ? (n - s0) : b.q_cap);
-        vs.resize(m);
-        for (uint32_t k = 0; k < m; k++) {
-            if (idx[s0 + k] >= c->cfg[inst].N) return set_err("potg_direct_sum: index out of range"), POTG_ERR_ARG;
-            vs[k] = inv[off + idx[s0 + k]];
-        }
-        HIPCHK(hipMemcpyAsync(b.q_self, vs.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
+        for (uint32_t k = 0; k < m; k++)
+            if (idx[s0 + k] >= p.N) return set_err("potg_direct_sum: index out of range"), POTG_ERR_ARG;
+        HIPCHK(hipMemcpyAsync(b.q_self, idx + s0, sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
+        launch_point_targets(b, inst, p.offset, p.N, m, 1, c->stream);
         launch_direct_sum(b, inst, (uint32_t)c->cfg[inst].N, m, c->stream);
         HIPCHK(hipMemcpyAsync(E + 3 * s0, b.q_out, 3 * sizeof(double) * m, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -1004,6 +986,12 @@ int potg_stats(potg_ctx* c, potg_stats_t* out)
     memset(out, 0, sizeof(*out));
     out->steps = g.n_steps;
     out->n_targets = g.n_tgt_total;
+    for (const auto& q : g.lone) {
+        g.n_cell += q.n[0];
+        g.n_leaf += q.n[1];
+        g.n_open += q.n[2];
+        g.n_pops += q.n[3];
+    }
     out->n_cell = g.n_cell;
     out->n_leaf = g.n_leaf;
     out->n_open = g.n_open;
@@ -1051,6 +1039,7 @@ int potg_stats_reset(potg_ctx* c)
     Globals g;
     HIPCHK(hipMemcpy(&g, c->b.g, sizeof(g), hipMemcpyDeviceToHost));
     g.n_cell = g.n_leaf = g.n_open = g.n_tgt_total = g.n_steps = g.n_pops = g.n_visits = 0;
+    memset(g.lone, 0, sizeof(g.lone));
     g.max_depth = 0;
     HIPCHK(hipMemcpy(c->b.g, &g, sizeof(g), hipMemcpyHostToDevice));
     return POTG_OK;
@@ -1187,6 +1176,7 @@ int potg_tune(potg_ctx* c, potg_tuning* out)
     g1.n_leaf = g0.n_leaf;
     g1.n_open = g0.n_open;
     g1.n_pops = g0.n_pops;
+    memcpy(g1.lone, g0.lone, sizeof(g1.lone));
     g1.n_visits = g0.n_visits;
     g1.n_tgt_total = g0.n_tgt_total;
     g1.n_steps = g0.n_steps;

@@ -154,6 +154,10 @@ void launch_init_slots(Bufs& b, hipStream_t s);
 void launch_unsort(Bufs& b, hipStream_t s);
 // point queries: n points of q_pts with q_inst/q_self; kind 0 field, 1 potential
 void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s);
+// q_inst of n points, and q_self: from the reference indexes that it holds (of
+// N particles from `offset`; larger ones are none), or none without `indexes`
+void launch_point_targets(Bufs& b, uint32_t inst, uint32_t offset, uint32_t N, uint32_t n,
+                          int indexes, hipStream_t s);
 // n_src: particles of the instance (its grain included)
 void launch_direct_sum(Bufs& b, uint32_t inst, uint32_t n_src, uint32_t n, hipStream_t s);
 // potg_phi_at_noalloc: this device's scratch array (0 on success), and the

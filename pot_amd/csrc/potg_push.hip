@@ -952,6 +952,17 @@ __global__ void k_inverse(PState st, uint32_t n, uint32_t* __restrict__ inv)
     if (r < n) inv[r] = i;
 }
 
+__global__ void k_point_targets(const uint32_t* __restrict__ inv, uint32_t inst, uint32_t offset,
+                                uint32_t N, uint32_t n, int indexes, uint32_t* __restrict__ q_inst,
+                                uint32_t* q_self)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    q_inst[i] = inst;
+    const uint32_t e = indexes ? q_self[i] : NONE;
+    q_self[i] = e < N ? inv[offset + e] : NONE;
+}
+
 // every slot starts as itself: reference layout, owned by its instance
 __global__ void k_init_slots(PState st, const InstParams* __restrict__ P, uint32_t n_inst,
                              uint32_t n)
@@ -1157,6 +1168,12 @@ void launch_gather_download(Bufs& b, uint32_t inst, uint32_t offset, double* aos
 void launch_build_inverse(Bufs& b, hipStream_t s)
 {
     k_inverse<<<grid(b.n_total), BT, 0, s>>>(b.st, b.n_total, b.inv);
+}
+
+void launch_point_targets(Bufs& b, uint32_t inst, uint32_t offset, uint32_t N, uint32_t n, int indexes,
+                          hipStream_t s)
+{
+    if (n) k_point_targets<<<grid(n), BT, 0, s>>>(b.inv, inst, offset, N, n, indexes, b.q_inst, b.q_self);
 }
 
 void launch_init_slots(Bufs& b, hipStream_t s)

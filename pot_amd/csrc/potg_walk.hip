@@ -1055,21 +1055,26 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
     const uint32_t ci = lane & 7u;
     const uint2* const s_top = s_stk - 1 - (lane >> 3);  // the lane's range at sp = 0
     const uint32_t ntg = (MODE == MODE_STEP) ? *io.n_targets_dev : io.n_pts;
-    if (rfl(step_failed(g) ? 1u : 0u)) return;
+    const bool failed = rfl(step_failed(g) ? 1u : 0u) != 0u;
     if (lane < 8u) s_mem[wv][lane] = make_uint2(0u, 0u);
+    __shared__ unsigned long long s_tot[4];
+    if constexpr (COUNT && KIND == KIND_FIELD) {
+        if (threadIdx.x < 4u) s_tot[threadIdx.x] = 0ull;
+        __syncthreads();
+    }
     unsigned long long tot_cell = 0, tot_leaf = 0, tot_open = 0, tot_pops = 0;
     const uint32_t nblk = (ntg + NW * per_wave - 1) / (NW * per_wave);
     const uint32_t per_xcd = (nblk + XCDS - 1) / XCDS;
 
-    for (uint32_t b = blockIdx.x; b / XCDS < per_xcd; b += gridDim.x) {
+    for (uint32_t b = blockIdx.x; !failed && b / XCDS < per_xcd; b += gridDim.x) {
         const uint32_t tile = (b % XCDS) * per_xcd + b / XCDS;
         if (tile >= nblk) continue;
         // the wavefront's targets, one a lane
         const uint32_t k0 = (tile * NW + wv) * per_wave;
         uint32_t l_inst, l_self;
         double l_x, l_y, l_z;
-        const bool valid = load_target<MODE, F64 && MODE != MODE_POINTS>(P, st, io, k0 + lane, lane < per_wave ? ntg : 0u, l_inst,
-                                             l_self, l_x, l_y, l_z);
+        const bool valid = load_target<MODE, F64 && MODE != MODE_POINTS>(
+            P, st, io, k0 + lane, lane < per_wave ? ntg : 0u, l_inst, l_self, l_x, l_y, l_z);
         float l_fx = 0.f, l_fy = 0.f, l_fz = 0.f, l_soft2 = 0.f;
         if constexpr (!F64) {
             const InstParams& p = P[l_inst];
@@ -1308,18 +1313,21 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
             }
         }
     }
-    if (COUNT && KIND == KIND_FIELD) {
+    if constexpr (COUNT && KIND == KIND_FIELD) {
         for (int d = 1; d < WAVE; d <<= 1) {
             tot_cell += __shfl_xor(tot_cell, d, WAVE);
             tot_leaf += __shfl_xor(tot_leaf, d, WAVE);
             tot_open += __shfl_xor(tot_open, d, WAVE);
         }
         if (lane == 0) {
-            atomicAdd(&g->n_cell, tot_cell);
-            atomicAdd(&g->n_leaf, tot_leaf);
-            atomicAdd(&g->n_open, tot_open);
-            atomicAdd(&g->n_pops, tot_pops);
+            atomicAdd(&s_tot[0], tot_cell);
+            atomicAdd(&s_tot[1], tot_leaf);
+            atomicAdd(&s_tot[2], tot_open);
+            atomicAdd(&s_tot[3], tot_pops);
         }
+        __syncthreads();
+        if (threadIdx.x < 4u)
+            atomicAdd(&g->lone[blockIdx.x % LONE_SLOTS].n[threadIdx.x], s_tot[threadIdx.x]);
     }
 }
 
