@@ -199,19 +199,23 @@ void fill_params(InstParams& p, const potg_config& k)
 // since neighbours' sets then differ less, and the larger the tree, whose
 // nodes a few targets fetch from further away -- but a tile of 64 is a long
 // walk, too few of which keep a device below half a million particles busy to
-// the end.  Step walk, ms, 2 / 64 targets, for DIPOLES (monopoles cross over
-// about 0.03 lower in theta):
-//   theta  150k       500k       1M         2M
-//   0.14   4.5/15.6   24.5/27.1  60/43      146/79
-//   0.20   2.0/8.2    9.1/13.7   21.5/20.5  50/38
-//   0.25   1.2/5.5    4.9/8.6    11.0/12.9  25/24
-//   0.30   0.8/3.9    3.0/5.9    6.4/8.8    14/16
-// so the crossing is put at theta = c + 0.05 log2(N / 1M).  By an instance's
-// own values, so that its walk is the same alone and in a batch.
-int lone64_rule(const InstParams& p)
+// the end, also when four wavefronts share it.  Step walk, ms, 2 / 64 / 64 in
+// four parts, for DIPOLES (monopoles cross over about 0.03 lower in theta):
+//   theta  150k           500k            1M         2M
+//   0.14   4.3/15.9/9.5   24.5/27.2/23.2  60/43/40   146/80/77
+//   0.20   2.0/8.2        9.1/13.7        21.5/20.5  50/38
+//   0.25   1.2/5.5        4.6/8.7/8.5     11.0/12.9  24.4/24.3/24.0
+//   0.30   0.8/3.9        3.0/5.9         6.4/8.8    14/16
+// so the crossing is put at theta = c + 0.05 log2(N / 1M).  The parts' sums
+// take 96 bytes a particle, for a gain that goes down with the size: up to 32M
+// particles.  By an instance's own values, so that its walk is the same alone
+// and in a batch.
+int kind64_rule(const InstParams& p)
 {
-    if (p.tree_n < 500000u) return 1;
-    return sqrt(p.theta2) >= (p.dipoles ? 0.21 : 0.18) + 0.05 * log2((double)p.tree_n / 1e6);
+    if (p.tree_n < 500000u ||
+        sqrt(p.theta2) >= (p.dipoles ? 0.21 : 0.18) + 0.05 * log2((double)p.tree_n / 1e6))
+        return KIND64_FEW;
+    return p.tree_n < 32000000u ? KIND64_SPLIT : KIND64_TILE;
 }
 
 // chi_b sampling point of the one worker (measure_chi_b, pot.c:2257-2275)
@@ -461,8 +465,8 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
         c->hp[i].offset = off;
         c->hp[i].tree_begin = tb;
         c->hp[i].tree_n = (uint32_t)configs[i].N - (configs[i].geometry != POTG_SPHERE ? 1 : 0);
-        c->hp[i].lone64 = lone64_rule(c->hp[i]);
-        b.n_lone64 += c->hp[i].lone64 != 0;
+        c->hp[i].kind64 = kind64_rule(c->hp[i]);
+        b.n_kind64[c->hp[i].kind64]++;
         b.any_bare |= c->hp[i].tree_n <= 1;
         off += (uint32_t)configs[i].N;
         tb += c->hp[i].tree_n;
@@ -528,6 +532,7 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
     rc |= alloc_n(c, &b.t_first, n_inst) | alloc_n(c, &b.t_base, n_inst);
     rc |= alloc_n(c, &b.queue, nt);
     rc |= alloc_n(c, &b.E, 3 * tc) | alloc_n(c, &b.inv, n);
+    if (precision == POTG_FP64 && b.n_kind64[KIND64_SPLIT]) rc |= alloc_n(c, &b.parts, 3 * SPLIT64 * tc);
     b.integrator = configs[0].integrator;
     if (b.integrator != POTG_BORIS) rc |= alloc_n(c, &b.a1, 3 * tc) | alloc_n(c, &b.x0, 3 * tc);
     bool any_bounce = false;

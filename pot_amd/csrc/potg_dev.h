@@ -24,6 +24,8 @@ constexpr uint32_t LEAF = 0xFFFFFFFFu;   // NodeRec.cnt marker of a leaf
 constexpr uint32_t NONE = 0xFFFFFFFFu;
 constexpr uint32_t LEAF_BIT = 0x80000000u; // child-slot code of a leaf
 constexpr int WAVE = 64;
+// float64 walk: 64 targets a wavefront, few, or 64 shared by SPLIT64 wavefronts
+constexpr int KIND64_TILE = 0, KIND64_FEW = 1, KIND64_SPLIT = 2, SPLIT64 = 4;
 constexpr int EPE_BLOCKS = 64;    // partial sums per instance of the PE reduction
 // tree moments by level: blocks of the depth counting sort, and the band of
 // depths given a launch per level (the others are done by one block)
@@ -74,7 +76,7 @@ struct InstParams {
     int32_t integrator;    // POTG_BORIS / POTG_VERLET / POTG_EULER_RICHARDSON
     int32_t out_bounce;    // OUT_BOUNCE: bounce off the wall
     double bounce_coe;     // its coefficient of restitution
-    int32_t lone64;        // the float64 walk has few targets a wavefront
+    int32_t kind64;        // KIND64_*: the shape of the float64 walk
 };
 
 // Mutable per-instance state on the device.

@@ -57,15 +57,16 @@ struct WalkIO {
     const InstState* S;
     const double* dip64;   // record dipoles (DIPOLES instances), else null
     const float4* dip32;
-    // the targets of every instance (PICK_ALL), or of those whose float64 walk
-    // has few targets a wavefront (InstParams::lone64), or 64
+    // the targets of the instances whose float64 walk is of this kind
+    // (InstParams::kind64), or of all (PICK_ALL)
     int32_t pick;
+    double* parts;     // a split float64 walk's partial sums
 };
-enum { PICK_ALL = 0, PICK_LONE = 1, PICK_SHARED = 2 };
+constexpr int32_t PICK_ALL = -1;
 
 __device__ inline bool picked(const InstParams& p, int32_t pick)
 {
-    return pick == PICK_ALL || (p.lone64 != 0) == (pick == PICK_LONE);
+    return pick == PICK_ALL || p.kind64 == pick;
 }
 
 __device__ inline void kahan_add(float& s, float& c, float v)
@@ -174,7 +175,19 @@ struct Staged64 {
     uint32_t first, cnt, part, pad;
 };
 
-template <int MODE, int KIND, bool DIP, bool COUNT>
+// the children that part `part` of SPLIT takes of the range below child j
+template <int SPLIT>
+__device__ inline uint32_t part_share(uint32_t part, uint32_t j)
+{
+    static_assert(SPLIT == 1 || SPLIT == 4, "a pattern of 8 / SPLIT children");
+    return SPLIT == 1 ? 0xffu : (0x11u << ((part - j) & 3u)) & 0xffu;
+}
+
+// SPLIT: wavefronts that share a tile, each a part of the cells two levels
+// below the root (k_sum_parts adds their sums): with 500k particles a tile a
+// wavefront leaves the device half empty at the end, DIPOLES at theta 0.14
+// 27.2 ms, in four parts 23.2 (1M particles 43.4 and 40.2, 2M 79.6 and 76.7)
+template <int MODE, int KIND, bool DIP, bool COUNT, int SPLIT>
 __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P, Globals* g,
                                                 PState st, const NodeRec64* __restrict__ rec,
                                                 WalkIO io)
@@ -189,9 +202,10 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
     unsigned long long tot_cell = 0, tot_leaf = 0, tot_open = 0, tot_pops = 0;
 
     for (;;) {
-        uint32_t tile = 0;
-        if (lane == 0) tile = atomicAdd(io.tile_ctr, 1u);
-        tile = rfl(__shfl(tile, 0, WAVE));
+        uint32_t item = 0;
+        if (lane == 0) item = atomicAdd(io.tile_ctr, 1u);
+        item = rfl(__shfl(item, 0, WAVE));
+        const uint32_t tile = item / SPLIT, part = item % SPLIT;
         if ((uint64_t)tile * WAVE >= ntg || rfl(step_failed(g) ? 1u : 0u)) break;
         const uint32_t k = tile * WAVE + lane;
         uint32_t inst, self;
@@ -209,6 +223,10 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
             if (rfl(P[gi].tree_n) == 0u) continue;  // no nodes
             const double theta2 = P[gi].theta2, soft2 = P[gi].soft2;
             const bool dip = DIP && P[gi].dipoles && io.dip64;
+            // the root's children, taken by part 0 and descended by all; of
+            // theirs a part takes its share of every range
+            const uint32_t rf = SPLIT > 1 ? rfl(rec[gi].first) : 0u;
+            uint32_t share = 0xffu;
             // the range to sweep next: the root's
             uint32_t tf = gi, tc = 1;
             uint64_t tm = grp;
@@ -248,8 +266,9 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
                     chg = (uint32_t)ballot((DIP && dip) ? r.part != 0u : r.q != 0) & inm;
                 }
                 __builtin_amdgcn_wave_barrier();
-                const uint32_t all = (1u << tc) - 1u;
-                const uint32_t lv = all & lm, cl = all & ~lm;
+                const bool top = SPLIT > 1 && (tf == gi || tf == rf) && part != 0u;
+                const uint32_t all = ((1u << tc) - 1u) & share;
+                const uint32_t lv = top ? 0u : all & lm, cl = all & ~lm;
                 for (uint32_t m = lv; m; m &= m - 1u) {
                     const Staged64& r = s_rec[wv][__builtin_ctz(m)];
                     const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
@@ -287,9 +306,9 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
                     const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
                     const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
                     const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
-                    const uint64_t m_use = tm & m_acc, m_open = tm & ~m_acc;
+                    const uint64_t m_use = top ? 0ull : tm & m_acc, m_open = tm & ~m_acc;
                     if (m_open) {
-                        if (COUNT) nopen += lane_of(m_open) ? 1u : 0u;
+                        if (COUNT && !top) nopen += lane_of(m_open) ? 1u : 0u;
                         if (!opened) om = m_open;
                         opened |= 1u << j;
                     }
@@ -358,6 +377,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
                     s_mask[wv][sp] = tm;
                     sp++;
                 }
+                if (SPLIT > 1) share = tf == rf ? part_share<SPLIT>(part, j) : 0xffu;
                 tf = next_first;
                 tc = next_cnt;
                 tm = om;
@@ -365,7 +385,12 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
         }
         if (valid) {
             const double K = QE / K4PE0;
-            if (KIND == KIND_FIELD) {
+            if (SPLIT > 1) {
+                double* o = io.parts + 3 * ((size_t)part * ntg + k);
+                o[0] = ex;
+                o[1] = ey;
+                o[2] = ez;
+            } else if (KIND == KIND_FIELD) {
                 io.out[3 * k] = (io.acc ? io.out[3 * k] : 0.0) + K * ex;
                 io.out[3 * k + 1] = (io.acc ? io.out[3 * k + 1] : 0.0) + K * ey;
                 io.out[3 * k + 2] = (io.acc ? io.out[3 * k + 2] : 0.0) + K * ez;
@@ -389,6 +414,23 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
             atomicAdd(&g->n_open, tot_open);
             atomicAdd(&g->n_pops, tot_pops);
         }
+    }
+}
+
+// the sums of the wavefronts that shared the targets' tiles
+template <int SPLIT>
+__global__ __launch_bounds__(BT) void k_sum_parts(const InstParams* __restrict__ P, PState st, WalkIO io)
+{
+    const uint32_t k = blockIdx.x * BT + threadIdx.x, ntg = *io.n_targets_dev;
+    if (k >= ntg) return;
+    const uint32_t i = io.targets[k];
+    if (i == NONE || !picked(P[st.inst[i]], io.pick)) return;
+    const double K = QE / K4PE0;
+    for (int d = 0; d < 3; d++) {
+        double e = 0.0;
+#pragma unroll
+        for (int p = 0; p < SPLIT; p++) e += io.parts[3 * ((size_t)p * ntg + k) + d];
+        io.out[3 * (size_t)k + d] = (io.acc ? io.out[3 * (size_t)k + d] : 0.0) + K * e;
     }
 }
 
@@ -951,7 +993,7 @@ __global__ __launch_bounds__(BT) void k_walk32s(const InstParams* __restrict__ P
 // ---- 1 or 2 targets per wavefront, 64 nodes at once -------------------------
 //
 // Point queries of both precisions, the potential-energy walk and, where few
-// targets a wavefront are the faster shape (lone64), the float64 step walk.
+// targets a wavefront are the faster shape (KIND64_FEW), the float64 step walk.
 // (The float32 step walks keep k_walkg's and k_walk32s's order of summation.)
 //
 // The 64 lanes of a wavefront hold 64 nodes: up to 8 child ranges are taken
@@ -1820,6 +1862,8 @@ static WalkIO step_io(Bufs& b)
     io.n_targets_dev = &b.g->n_targets;
     io.out = b.E;
     io.acc = b.any_spheroid;
+    io.pick = PICK_ALL;
+    io.parts = b.parts;
     io.tile_ctr = &b.g->tile_ctr;
     io.n_rec = b.n_rec;
     io.dip64 = b.dip64;
@@ -1907,28 +1951,37 @@ static void launch_walk32(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
     else launch_walk32c<MODE, false>(b, blocks, io, s);
 }
 
-template <int MODE, int KIND, bool COUNT>
-static void launch_walk64c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
+template <int MODE, int KIND, bool COUNT, int SPLIT>
+static void launch_walk64s(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
 {
     if (b.dip64)
-        k_walk64<MODE, KIND, true, COUNT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, b.rec64, io);
+        k_walk64<MODE, KIND, true, COUNT, SPLIT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, b.rec64, io);
     else
-        k_walk64<MODE, KIND, false, COUNT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, b.rec64, io);
+        k_walk64<MODE, KIND, false, COUNT, SPLIT><<<blocks, BT, 0, s>>>(b.P, b.g, b.st, b.rec64, io);
 }
 
-// float64 walk: the instances that walk alone and those that walk together,
-// each by its kernel; `blocks` for the latter
+// float64 walk: the instances of each kind by their kernel; `blocks` for those
+// of 64 targets a wavefront
 template <int MODE, int KIND, bool COUNT>
 static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream_t s)
 {
-    const bool all = b.n_lone64 == b.n_inst;
-    if (b.n_lone64) {
-        io.pick = all ? PICK_ALL : PICK_LONE;
-        launch_walk1<MODE == MODE_STEP ? 2 : 1, true, MODE, KIND, COUNT>(b, n, io, s);
-    }
-    if (!all) {
-        io.pick = b.n_lone64 ? PICK_SHARED : PICK_ALL;
-        launch_walk64c<MODE, KIND, COUNT>(b, blocks, io, s);
+    const auto pick = [&](int kind) {
+        io.pick = b.n_kind64[kind] == b.n_inst ? PICK_ALL : kind;
+        return b.n_kind64[kind] != 0;
+    };
+    if (pick(KIND64_FEW)) launch_walk1<MODE == MODE_STEP ? 2 : 1, true, MODE, KIND, COUNT>(b, n, io, s);
+    if (pick(KIND64_TILE)) launch_walk64s<MODE, KIND, COUNT, 1>(b, blocks, io, s);
+    if (pick(KIND64_SPLIT)) {
+        if (b.n_kind64[KIND64_TILE]) k_reset_tiles<<<1, 1, 0, s>>>(io.tile_ctr);
+        if constexpr (MODE == MODE_STEP && KIND == KIND_FIELD) {
+            // more, shorter items: 8 blocks a CU where the tiles had fewer
+            const int most = 8 * device_cus();
+            if (blocks < most) blocks = 2 * blocks < most ? 2 * blocks : most;
+            launch_walk64s<MODE, KIND, COUNT, SPLIT64>(b, blocks, io, s);
+            k_sum_parts<SPLIT64><<<(b.t_cap + BT - 1) / BT, BT, 0, s>>>(b.P, b.st, io);
+        } else {
+            launch_walk64s<MODE, KIND, COUNT, 1>(b, blocks, io, s);
+        }
     }
 }
 
