@@ -2085,55 +2085,101 @@ void launch_epe(Bufs& b, hipStream_t s)
 }
 
 // chi_b every 20 steps (pot.c:2409-2418): the potential at one boundary
-// point per instance, before any particle moves; one lane walks (a handful
-// of nodes at the domain edge)
+// point per instance, before any particle moves.  A wavefront an instance: a
+// lane a child of the range, whose terms are then added one by one in the
+// order of the serial walk (children from the last to the first, an opened
+// one's before the next), so the sum is the serial one bit for bit.  Bound by
+// the loads, one range after the other: 96 us at 16k particles, 39 at 150k; by
+// one lane, a node after the other, 223 and 99.
 __global__ __launch_bounds__(64) void k_chi_b(const InstParams* __restrict__ P, InstState* S,
                                               Globals* g, const NodeRec64* __restrict__ r64,
                                               const double* __restrict__ dip64, uint32_t n_inst,
                                               uint32_t n_rec)
 {
+    __shared__ double s_term[STK][8];
+    __shared__ uint32_t s_cf[STK][8], s_cc[STK][8];
+    __shared__ uint32_t s_first[STK], s_todo[STK], s_mask[STK];
     if ((g->t % 20) != 0 || step_failed(g)) return;
-    const uint32_t inst = blockIdx.x;
-    if (inst >= n_inst || threadIdx.x != 0 || S[inst].retired) return;
+    const uint32_t inst = blockIdx.x, lane = threadIdx.x;
+    if (inst >= n_inst || S[inst].retired) return;
     const InstParams& p = P[inst];
     const double x = p.chi_pt[0], y = p.chi_pt[1], z = p.chi_pt[2];
     const double theta2 = p.theta2, soft2 = p.soft2;
+    const bool dip = p.dipoles && dip64;
     double ph = (p.geometry != 0) ? grain_phi_abs(p, S[inst].grain_q, x, y, z) : 0.0;
-    uint32_t stk[8 * STK];
-    int sp = 0;
-    stk[sp++] = inst;
-    uint32_t pops = 0;
-    while (sp) {
-        if (++pops > n_rec) {
-            raise_err(g, KERR_DEPTH, inst);
+    uint32_t first = inst, cnt = 1, loads = 0;  // the range to load
+    int d = 0;
+    for (;;) {
+        if (++loads > n_rec || cnt > 8u || d >= STK) {
+            if (lane == 0) raise_err(g, KERR_DEPTH, first);
             return;
         }
-        const uint32_t w = stk[--sp];
-        const NodeRec64 r = r64[w];
-        const double dx = x - r.cx, dy = y - r.cy, dz = z - r.cz;
-        const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
-        if (r.cnt == LEAF) {
-            ph += (QE * r.q) / (K4PE0 * sqrt(d2 + soft2));
-        } else if (r.size2 < theta2 * d2) {
-            if (p.dipoles && dip64) {
-                if (r.part) {  // |q| of the cell (pot.c:1856-1862)
-                    const double* d = dip64 + 3 * (size_t)w;
-                    const double dist = sqrt(d2);
-                    const double rdp = (dx * d[0]) + (dy * d[1]) + (dz * d[2]);
-                    ph += (QE / K4PE0) * ((r.q / dist) + (rdp / (dist * d2)));
+        bool adds = false, opens = false;
+        if (lane < cnt) {
+            const uint32_t w = first + lane;
+            const NodeRec64 r = r64[w];
+            const double dx = x - r.cx, dy = y - r.cy, dz = z - r.cz;
+            const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
+            double term = 0.0;
+            if (r.cnt == LEAF) {
+                adds = true;
+                term = (QE * r.q) / (K4PE0 * sqrt(d2 + soft2));
+            } else if (r.size2 < theta2 * d2) {
+                if (dip) {
+                    if (r.part) {  // |q| of the cell (pot.c:1856-1862)
+                        const double* m = dip64 + 3 * (size_t)w;
+                        const double dist = sqrt(d2);
+                        const double rdp = (dx * m[0]) + (dy * m[1]) + (dz * m[2]);
+                        adds = true;
+                        term = (QE / K4PE0) * ((r.q / dist) + (rdp / (dist * d2)));
+                    }
+                } else if (r.q) {
+                    adds = true;
+                    term = (QE * r.q) / (K4PE0 * sqrt(d2));
                 }
-            } else if (r.q) {
-                ph += (QE * r.q) / (K4PE0 * sqrt(d2));
+            } else {
+                opens = true;
             }
-        } else {
-            if (sp + (int)r.cnt > 8 * STK || (r.cnt && r.first <= w) || r.first + r.cnt > n_rec) {
-                raise_err(g, KERR_DEPTH, w);
+            s_term[d][lane] = term;
+            s_cf[d][lane] = r.first;
+            s_cc[d][lane] = r.cnt;
+        }
+        uint32_t todo = (uint32_t)ballot(adds || opens);
+        uint32_t open = (uint32_t)ballot(opens);
+        uint32_t f = first;
+        __builtin_amdgcn_wave_barrier();
+        cnt = 0;
+        for (;;) {
+            if (!todo) {
+                if (d == 0) break;
+                d--;
+                todo = rfl(s_todo[d]);
+                open = rfl(s_mask[d]);
+                f = rfl(s_first[d]);
+                continue;
+            }
+            const uint32_t j = 31u - (uint32_t)__builtin_clz(todo);
+            todo &= ~(1u << j);
+            if (!((open >> j) & 1u)) {
+                ph += s_term[d][j];
+                continue;
+            }
+            first = rfl(s_cf[d][j]);
+            cnt = rfl(s_cc[d][j]);
+            if (cnt == 0) continue;  // an empty cell
+            if (first <= f + j || first + cnt > n_rec) {
+                if (lane == 0) raise_err(g, KERR_DEPTH, f + j);
                 return;
             }
-            for (uint32_t c = 0; c < r.cnt; c++) stk[sp++] = r.first + c;
+            s_todo[d] = todo;
+            s_mask[d] = open;
+            s_first[d] = f;
+            d++;
+            break;
         }
+        if (cnt == 0) break;
     }
-    S[inst].chi_b = ph / p.kTi_over_e;
+    if (lane == 0) S[inst].chi_b = ph / p.kTi_over_e;
 }
 
 void launch_chi_b(Bufs& b, hipStream_t s)
