@@ -4,7 +4,7 @@
  * One context holds one or more independent grain simulations
  * ("instances") resident in HBM.  A step advances every instance by one
  * time step: octree build (Morton keys with the reference's float64
- * midpoint recurrence, radix sort, bottom-up octree, monopole moments),
+ * midpoint recurrence, merge or radix sort, bottom-up octree, moments),
  * Barnes-Hut field walk, Boris push, grain crossing with exact integer
  * tallies, and SCEPTIC-like reinjection from a counter-based stream.
  *
