@@ -304,8 +304,7 @@ void enqueue_step(potg_ctx* c, int compute_epe)
     Bufs& b = c->b;
     hipStream_t s = c->stream;
     record(c, 0);
-    launch_begin_step(b, s);
-    launch_keys_sort_permute(b, s);
+    launch_keys_sort_permute(b, true, s);
     record(c, 1);
     launch_tree(b, s);
     launch_targets(b, s);
@@ -779,7 +778,7 @@ int potg_build_tree(potg_ctx* c)
     if (!c) return set_err("potg_build_tree: null context"), POTG_ERR_ARG;
     if (all_uploaded(c)) return POTG_ERR_ARG;
     destroy_graphs(c);
-    launch_keys_sort_permute(c->b, c->stream);
+    launch_keys_sort_permute(c->b, false, c->stream);
     launch_tree(c->b, c->stream);
     HIPCHK(hipGetLastError());
     return kernel_error(c);
@@ -1089,8 +1088,7 @@ int potg_tune(potg_ctx* c, potg_tuning* out)
     Globals g0;
     HIPCHK(hipMemcpy(&g0, b.g, sizeof(g0), hipMemcpyDeviceToHost));
     // everything the coming step does before its walk
-    launch_begin_step(b, s);
-    launch_keys_sort_permute(b, s);
+    launch_keys_sort_permute(b, true, s);
     launch_tree(b, s);
     launch_targets(b, s);
     HIPCHK(hipStreamSynchronize(s));
@@ -1155,7 +1153,7 @@ int potg_tune(potg_ctx* c, potg_tuning* out)
             float ms_best = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
                 HIPCHK(hipEventRecord(e0, s));
-                launch_keys_sort_permute(b, s);
+                launch_keys_sort_permute(b, false, s);
                 HIPCHK(hipEventRecord(e1, s));
                 HIPCHK(hipEventSynchronize(e1));
                 float ms = 0.f;

@@ -124,8 +124,8 @@ struct Bufs {
 };
 
 // step stages (kernel launches only; no synchronisation)
-void launch_begin_step(Bufs& b, hipStream_t s);
-void launch_keys_sort_permute(Bufs& b, hipStream_t s);
+// begin: a step begins with it (step counter, tallies, work counters)
+void launch_keys_sort_permute(Bufs& b, bool begin, hipStream_t s);
 void launch_tree(Bufs& b, hipStream_t s);
 void launch_targets(Bufs& b, hipStream_t s);
 void launch_chi_b(Bufs& b, hipStream_t s);

@@ -67,10 +67,12 @@ __device__ inline int split_depth(double ax, double ay, double az, double bx, do
 }
 
 // ---------------------------------------------------------------------
-// One block: every thread reads the step counter before thread 0 advances
-// it (the barrier), however many instances there are.
-__global__ void k_begin_step(InstParams* __restrict__ P, InstState* __restrict__ S, Globals* g,
-                             uint32_t n_inst)
+// A new step begins, in the first block of the launch that computes its keys:
+// every thread reads the step counter before thread 0 advances it (the
+// barrier), however many instances there are.  Nothing else in that launch
+// reads what is written here.
+__device__ inline void begin_step(const InstParams* __restrict__ P, InstState* __restrict__ S,
+                                  Globals* g, uint32_t n_inst)
 {
     const uint64_t t = g->t + 1;  // the step being taken (pot.c:4261)
     for (uint32_t k = threadIdx.x; k < n_inst; k += blockDim.x) {
@@ -147,9 +149,12 @@ __device__ inline uint64_t key_of(uint32_t i, const InstParams* __restrict__ P, 
     return k;
 }
 
-__global__ void k_keys(const InstParams* __restrict__ P, PState st, uint32_t n, int levels,
-                       uint64_t* __restrict__ key, uint32_t* __restrict__ perm, Globals* g)
+// begins: the instances of the step that begins, or 0
+__global__ void k_keys(const InstParams* __restrict__ P, InstState* __restrict__ S, uint32_t begins,
+                       PState st, uint32_t n, int levels, uint64_t* __restrict__ key,
+                       uint32_t* __restrict__ perm, Globals* g)
 {
+    if (begins && blockIdx.x == 0) begin_step(P, S, g, begins);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     perm[i] = i;
@@ -157,12 +162,14 @@ __global__ void k_keys(const InstParams* __restrict__ P, PState st, uint32_t n, 
 }
 
 // the keys in sorted tiles
-__global__ __launch_bounds__(MERGE_TILE) void k_key_tiles(const InstParams* __restrict__ P, PState st,
-                                                          uint32_t n, int levels,
+__global__ __launch_bounds__(MERGE_TILE) void k_key_tiles(const InstParams* __restrict__ P,
+                                                          InstState* __restrict__ S, uint32_t begins,
+                                                          PState st, uint32_t n, int levels,
                                                           uint64_t* __restrict__ key,
                                                           uint32_t* __restrict__ perm, Globals* g)
 {
     __shared__ TileSort sh;
+    if (begins && blockIdx.x == 0) begin_step(P, S, g, begins);
     const uint32_t t0 = blockIdx.x * MERGE_TILE, i = t0 + threadIdx.x;
     // what fills the last tile sorts behind all
     uint64_t k = i < n ? key_of(i, P, st, levels, g) : ~0ull;
@@ -1283,11 +1290,6 @@ __global__ __launch_bounds__(1024) void k_level_moments_block(
 
 }  // namespace
 
-void launch_begin_step(Bufs& b, hipStream_t s)
-{
-    k_begin_step<<<1, BT, 0, s>>>(b.P, b.S, b.g, b.n_inst);
-}
-
 // the leaf records again, from the current state: between the two fields
 // of velocity Verlet / Euler-Richardson the reference's walk reads its leaves
 // from the live array, which then holds the intermediate state, while the
@@ -1301,16 +1303,17 @@ void launch_leaf_refresh(Bufs& b, hipStream_t s)
                                           b.precision ? b.dip32 : nullptr);
 }
 
-void launch_keys_sort_permute(Bufs& b, hipStream_t s)
+void launch_keys_sort_permute(Bufs& b, bool begin, hipStream_t s)
 {
-    const uint32_t n = b.n_total;
+    const uint32_t n = b.n_total, begins = begin ? b.n_inst : 0u;
     if (n < MERGE_MAX) {
         const bool alt = merge_passes(n) & 1;
         k_key_tiles<<<(n + MERGE_TILE - 1) / MERGE_TILE, MERGE_TILE, 0, s>>>(
-            b.P, b.st, n, b.key_levels, alt ? b.key_alt : b.key, alt ? b.perm_alt : b.perm, b.g);
+            b.P, b.S, begins, b.st, n, b.key_levels, alt ? b.key_alt : b.key,
+            alt ? b.perm_alt : b.perm, b.g);
         merge_tiles(b.key, b.key_alt, b.perm, b.perm_alt, n, s);
     } else {
-        k_keys<<<grid(n), BT, 0, s>>>(b.P, b.st, n, b.key_levels, b.key, b.perm, b.g);
+        k_keys<<<grid(n), BT, 0, s>>>(b.P, b.S, begins, b.st, n, b.key_levels, b.key, b.perm, b.g);
         radix_sort_pairs(b.key, b.key_alt, b.perm, b.perm_alt, n, b.key_bits, b.sort_tmp,
                          (int)b.sort_ipt, s);
     }
