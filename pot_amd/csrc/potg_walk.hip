@@ -1193,6 +1193,7 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
                     if constexpr (F64) r = rec[w];
                     else r = *(const Rec*)((const uint4*)rec + w);
                     const uint64_t m_leaf = ballot(r.cnt == LEAF);
+                    // cells are not softened
                     const float soft = !F64 && lane_of(m_leaf) ? soft2f : 0.f;
                     uint64_t m_open = 0;  // by any of the targets
                     uint32_t y = r.cnt;
@@ -1259,16 +1260,14 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
                             }
                         } else {
                             const float dx = tx[i] - r.cx, dy = ty[i] - r.cy, dz = tz[i] - r.cz;
-                            // softened for leaves; for cells the softening is
-                            // zero and d2 the plain squared distance.  A leaf's
-                            // size2 is zero: unsoftened at float32 distance
-                            // zero it is not taken, softened it adds zero
                             const float d2 =
-                                __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, soft)));
-                            const uint64_t m_acc = ballot(!(d2 <= r.size2));
-                            m_use = m_in & m_acc & ~m_own;
+                                __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+                            // a leaf at float32 distance zero adds nothing
+                            const uint64_t m_far = ballot(d2 != 0.f);
+                            const uint64_t m_acc = ballot(r.size2 < d2);
+                            m_use = m_in & ((m_leaf & m_far) | (m_acc & ~m_leaf)) & ~m_own;
                             m_op = m_in & ~(m_acc | m_leaf);
-                            const float inv = lane_of(m_use) ? __builtin_amdgcn_rsqf(d2) : 0.f;
+                            const float inv = lane_of(m_use) ? __builtin_amdgcn_rsqf(d2 + soft) : 0.f;
                             const float inv2 = inv * inv, inv3 = inv2 * inv;
                             if (DIP && dip) {
                                 const float rpd2 =
@@ -1287,10 +1286,7 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
                         if (COUNT) {
                             const uint64_t m_chg = ballot(dip ? r.part != 0u : r.q != 0);
                             ncell[i] += lane_of(m_use & ~m_leaf & m_chg) ? 1u : 0u;
-                            uint64_t m_far = ~0ull;  // a coincident leaf does not count
-                            if constexpr (!F64)
-                                m_far = ballot(tx[i] != r.cx || ty[i] != r.cy || tz[i] != r.cz);
-                            nleaf[i] += lane_of(m_use & m_leaf & m_far) ? 1u : 0u;
+                            nleaf[i] += lane_of(m_use & m_leaf) ? 1u : 0u;
                             nopen[i] += lane_of(m_op) ? 1u : 0u;
                         }
                         m_open |= m_op;
