@@ -1043,7 +1043,8 @@ __global__ __launch_bounds__(BT) void k_direct(const InstParams* __restrict__ P,
                  tz = valid ? st.z[self] : 0.0;
     // the target among the sources
     const uint32_t self_j = valid ? st.ref[self] - p.offset : NONE;
-    const double soft2 = p.soft2;
+    // (a softening whose square is infinite still gives zero, not NaN)
+    const double soft2 = __builtin_fmin(p.soft2, 0x1p1000);
     // the spheroid grain is analytic, not a point source (SPH:1516-1521)
     const uint32_t j_begin = p.geometry != 0 ? 1u : 0u;
     const uint32_t nchunk = (p.N - j_begin + BT - 1) / BT;

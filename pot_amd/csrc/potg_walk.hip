@@ -147,11 +147,13 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
 }
 
 // 1 / sqrt(r2) to the last bits: the hardware's value (relative error below
-// 2^-23), then (1 - e)^(-1/2) = 1 + e/2 + 3/8 e^2 + O(e^3), e = 1 - r2 r^2
+// 2^-23), then (1 - e)^(-1/2) = 1 + e/2 + 3/8 e^2 + O(e^3), e = 1 - r2 r^2.
+// r2 r is kept from becoming NaN at either end, where the result is 1 / 0 or
+// 1 / infinity (a point so far out that its squared distance overflows)
 __device__ inline double rsqrt64(double r2)
 {
     const double r = __builtin_amdgcn_rsq(r2);
-    const double e = __builtin_fma(-r2 * r, r, 1.0);
+    const double e = __builtin_fma(-__builtin_fmin(r2 * r, 0x1p1000), r, 1.0);
     return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
 }
 
@@ -284,9 +286,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
                         }
                     }
                     const double r2 = d2 + soft2;
-                    double inv = rsqrt64(r2);
-                    if (KIND != KIND_FIELD && r2 == 0.0) inv = __builtin_inf();
-                    inv = lane_of(m_use) ? inv : 0.0;
+                    const double inv = lane_of(m_use) ? rsqrt64(r2) : 0.0;
                     if (KIND == KIND_FIELD) {
                         const double ca = r.q * (inv * inv * inv);
                         ex = __builtin_fma(ca, dx, ex);
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
                     const Staged64& r = s_rec[wv][j];
                     const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
                     const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
-                    const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
+                    const uint64_t m_acc = ballot(r.size2 < theta2 * d2);
                     const uint64_t m_use = top ? 0ull : tm & m_acc, m_open = tm & ~m_acc;
                     if (m_open) {
                         if (COUNT && !top) nopen += lane_of(m_open) ? 1u : 0u;
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
                         const NodeRec64 r = rec[tf + j];
                         const double dx = tx - r.cx, dy = ty - r.cy, dz = tz - r.cz;
                         const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
-                        om = tm & ballot(theta2 * d2 <= r.size2);
+                        om = tm & ~ballot(r.size2 < theta2 * d2);
                         next_first = rfl(r.first);
                         next_cnt = rfl(r.cnt);
                     }
@@ -1218,7 +1218,7 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
                             const double dx = dtx[i] - r.cx, dy = dty[i] - r.cy, dz = dtz[i] - r.cz;
                             // the reference's opening test, in its operations
                             const double d2 = (dx * dx) + (dy * dy) + (dz * dz);
-                            const uint64_t m_acc = ballot(!(theta2 * d2 <= r.size2));
+                            const uint64_t m_acc = ballot(r.size2 < theta2 * d2);
                             m_use = m_in & (m_acc | m_leaf) & ~m_own;
                             if (KIND == KIND_FIELD) {
                                 const uint64_t m_hit = m_use & m_leaf & ballot(d2 == 0.0);
@@ -1230,9 +1230,7 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
                             m_op = m_in & ~(m_acc | m_leaf);
                             const bool use = lane_of(m_use);
                             const double r2 = lane_of(m_leaf) ? d2 + soft2 : d2;
-                            double inv = rsqrt64(r2);
-                            if (KIND != KIND_FIELD && r2 == 0.0) inv = __builtin_inf();
-                            inv = use ? inv : 0.0;
+                            const double inv = use ? rsqrt64(r2) : 0.0;
                             const double q = (double)r.q;
                             if (KIND == KIND_FIELD) {
                                 const double inv2 = inv * inv, inv3 = inv2 * inv;
