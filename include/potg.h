@@ -156,7 +156,8 @@ typedef struct potg_stats_t {
    below.  They concern step walks (point queries follow a group of 16 or
    variant 0 only) and, of the float64 ones, those of instances with 64
    targets per wavefront: an instance whose opening angle is large for its
-   size, or with less than half a million particles, is walked 2 by 2. */
+   size (DIPOLES: 0.15 at 0.5M particles, 0.2 at 1M, 0.25 at 2M) is walked 2
+   by 2. */
 typedef struct potg_tuning {
     uint32_t walk_blocks; /* blocks (4 wavefronts each) of the persistent walk */
     uint32_t group;       /* float32 walk: targets per wavefront, 8, 16 or 64;

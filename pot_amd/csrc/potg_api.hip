@@ -197,25 +197,55 @@ void fill_params(InstParams& p, const potg_config& k)
 // (k_walk64).  With few, hardly a lane works for another's target; 64 share
 // every node's load and its instructions, the better the smaller theta,
 // since neighbours' sets then differ less, and the larger the tree, whose
-// nodes a few targets fetch from further away -- but a tile of 64 is a long
-// walk, too few of which keep a device below half a million particles busy to
-// the end, also when four wavefronts share it.  Step walk, ms, 2 / 64 / 64 in
-// four parts, for DIPOLES (monopoles cross over about 0.03 lower in theta):
-//   theta  150k           500k            1M         2M
-//   0.14   4.3/15.9/9.5   24.5/27.2/23.2  60/43/40   146/80/77
-//   0.20   2.0/8.2        9.1/13.7        21.5/20.5  50/38
-//   0.25   1.2/5.5        4.6/8.7/8.5     11.0/12.9  24.4/24.3/24.0
-//   0.30   0.8/3.9        3.0/5.9         6.4/8.8    14/16
-// so the crossing is put at theta = c + 0.05 log2(N / 1M).  The parts' sums
-// take 96 bytes a particle, for a gain that goes down with the size: up to 32M
-// particles.  By an instance's own values, so that its walk is the same alone
-// and in a batch.
+// nodes a few targets fetch from further away.  But a tile of 64 is a long
+// walk, too few of which keep the device busy to the end below some million
+// particles: four wavefronts share one.  Step walk, ms, 2 targets / 64 in four
+// parts (/ 64 in one), for DIPOLES; monopoles cross over about 0.03 lower:
+//   theta  100k   150k     200k     300k     450k       500k
+//   0      39/34  88/54    153/77   411/150  1015/296
+//   0.035  30/27  60/40    101/55   231/90   483/154
+//   0.05   21/22  38/32    60/41    132/67   265/103
+//   0.07   12/17  21.5/23  33/29    66/44    125/65
+//   0.09   7.5/13 13/18    19/21    37/32    68/46
+//   0.11   5.0/11 8.4/14   12/17    23/25    40/34
+//   0.13   3.4/7.9 5.8/10  8.2/13   15/18    25.8/24.1
+//   0.14                                     21.3/21.0  24.7/23.2/27.2
+//   theta  1M             2M              4M       8M       16M
+//   0.14   60/40/43       146/77/80
+//   0.20   21.6/21.1      50/38
+//   0.25   11.0/12.9      24.4/24.0/24.3
+//   0.31                                  27/29
+//   0.33                                           47.8/47.9
+//   0.38                                                    67/72
+// so the crossing is put at theta = c + 0.05 log2(N / 1M), the parts' gain
+// over a whole tile goes down with the size, and their sums take 96 bytes a
+// particle: up to 32M particles.  By an instance's own values, so that its walk
+// is the same alone and in a batch.
 int kind64_rule(const InstParams& p)
 {
-    if (p.tree_n < 500000u ||
-        sqrt(p.theta2) >= (p.dipoles ? 0.21 : 0.18) + 0.05 * log2((double)p.tree_n / 1e6))
+    if (sqrt(p.theta2) >= (p.dipoles ? 0.201 : 0.171) + 0.05 * log2((double)p.tree_n / 1e6))
         return KIND64_FEW;
     return p.tree_n < 32000000u ? KIND64_SPLIT : KIND64_TILE;
+}
+
+// The same for the potential-energy walk, which has one target a wavefront (no
+// pairs, which would depend on where an instance's slots start in a batch) or
+// 64 that one wavefront walks, and twice the targets.  ms, 1 target / 64:
+//   theta  50k      100k     200k     450k     1M       2M       4M
+//   0      23.2/22.8
+//   0.04   20/24*   69/41                               * 0.03
+//   0.07   11/19*   30/28    73/44**                    * 0.06  ** 0.08
+//   0.10            14/18    54/35*                     * 0.09
+//   0.15                     13.8/14.6 45/29
+//   0.20                              27/19.5* 52/27    * 0.18
+//   0.24                              11.0/10.6
+//   0.30                                       17/13*   30/20    81/42  * 0.29
+// and monopoles 200k 0.06 72/53, 0.09 30/30, 1M 0.23 19.5/15.7, 0.26 13.4/12.8,
+// 4M 0.39 21/18; before, with lane reads and divisions, 450k 0.15 took 60.
+int kind64_epe_rule(const InstParams& p)
+{
+    const double line = (p.dipoles ? 0.145 : 0.09) + 0.065 * log2((double)p.tree_n / 2e5);
+    return sqrt(p.theta2) >= line ? KIND64_FEW : KIND64_TILE;
 }
 
 // chi_b sampling point of the one worker (measure_chi_b, pot.c:2257-2275)
@@ -465,7 +495,9 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
         c->hp[i].tree_begin = tb;
         c->hp[i].tree_n = (uint32_t)configs[i].N - (configs[i].geometry != POTG_SPHERE ? 1 : 0);
         c->hp[i].kind64 = kind64_rule(c->hp[i]);
+        c->hp[i].kind64_epe = kind64_epe_rule(c->hp[i]);
         b.n_kind64[c->hp[i].kind64]++;
+        b.n_epe64[c->hp[i].kind64_epe]++;
         b.any_bare |= c->hp[i].tree_n <= 1;
         off += (uint32_t)configs[i].N;
         tb += c->hp[i].tree_n;

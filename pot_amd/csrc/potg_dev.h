@@ -76,7 +76,8 @@ struct InstParams {
     int32_t integrator;    // POTG_BORIS / POTG_VERLET / POTG_EULER_RICHARDSON
     int32_t out_bounce;    // OUT_BOUNCE: bounce off the wall
     double bounce_coe;     // its coefficient of restitution
-    int32_t kind64;        // KIND64_*: the shape of the float64 walk
+    int32_t kind64;        // KIND64_*: the shape of the float64 step walk
+    int32_t kind64_epe;    // and of the potential-energy walk (TILE or FEW)
 };
 
 // Mutable per-instance state on the device.

@@ -53,7 +53,7 @@ struct Bufs {
     int precision;     // POTG_FP64 / POTG_MIXED / POTG_MIXED_GROUP
     int any_spheroid;  // some instance has the analytic spheroid grain
     int any_bare;      // some instance's tree has no internal nodes
-    uint32_t n_kind64[3];  // instances by kind64
+    uint32_t n_kind64[3], n_epe64[3];  // instances by kind64 and kind64_epe
     double* parts;     // partial sums of the float64 walk's shared tiles
     int count;         // step walks keep the interaction counters (potg_set_counting)
     int key_levels;    // digits carried by a sort key

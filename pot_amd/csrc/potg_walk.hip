@@ -58,15 +58,15 @@ struct WalkIO {
     const double* dip64;   // record dipoles (DIPOLES instances), else null
     const float4* dip32;
     // the targets of the instances whose float64 walk is of this kind
-    // (InstParams::kind64), or of all (PICK_ALL)
+    // (InstParams::kind64, kind64_epe), or of all (PICK_ALL)
     int32_t pick;
     double* parts;     // a split float64 walk's partial sums
 };
 constexpr int32_t PICK_ALL = -1;
 
-__device__ inline bool picked(const InstParams& p, int32_t pick)
+__device__ inline bool picked(int32_t kind, int32_t pick)
 {
-    return pick == PICK_ALL || p.kind64 == pick;
+    return pick == PICK_ALL || kind == pick;
 }
 
 __device__ inline void kahan_add(float& s, float& c, float v)
@@ -112,7 +112,7 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
         if (i == NONE) return false;  // the gap before the next instance's targets
         self = i;
         inst = st.inst[i];
-        if (PICK && !picked(P[inst], io.pick)) return false;
+        if (PICK && !picked(P[inst].kind64, io.pick)) return false;
         if (P[inst].integrator == 0) {
             const double dts = P[inst].dt * (double)P[inst].tss[st.spec[i]];
             tx = st.x[i] + (0.5 * dts) * st.vx[i];
@@ -126,7 +126,7 @@ __device__ inline bool load_target(const InstParams* __restrict__ P, PState st, 
     } else if (MODE == MODE_EPE) {
         self = k;
         inst = st.inst[k];
-        if (PICK && !picked(P[inst], io.pick)) return false;
+        if (PICK && !picked(P[inst].kind64_epe, io.pick)) return false;
         const int sp = st.spec[k];
         // Boris half-drifted the stepped particles in place; the other
         // integrators' state already holds the intermediate state
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(BT) void k_sum_parts(const InstParams* __restrict__
     const uint32_t k = blockIdx.x * BT + threadIdx.x, ntg = *io.n_targets_dev;
     if (k >= ntg) return;
     const uint32_t i = io.targets[k];
-    if (i == NONE || !picked(P[st.inst[i]], io.pick)) return;
+    if (i == NONE || !picked(P[st.inst[i]].kind64, io.pick)) return;
     const double K = QE / K4PE0;
     for (int d = 0; d < 3; d++) {
         double e = 0.0;
@@ -1959,23 +1959,21 @@ static void launch_walk64s(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
 template <int MODE, int KIND, bool COUNT>
 static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream_t s)
 {
+    const uint32_t* n_kind = MODE == MODE_EPE ? b.n_epe64 : b.n_kind64;
     const auto pick = [&](int kind) {
-        io.pick = b.n_kind64[kind] == b.n_inst ? PICK_ALL : kind;
-        return b.n_kind64[kind] != 0;
+        io.pick = n_kind[kind] == b.n_inst ? PICK_ALL : kind;
+        return n_kind[kind] != 0;
     };
     if (pick(KIND64_FEW)) launch_walk1<MODE == MODE_STEP ? 2 : 1, true, MODE, KIND, COUNT>(b, n, io, s);
     if (pick(KIND64_TILE)) launch_walk64s<MODE, KIND, COUNT, 1>(b, blocks, io, s);
-    if (pick(KIND64_SPLIT)) {
+    if constexpr (MODE == MODE_STEP) {
+        if (!pick(KIND64_SPLIT)) return;
         if (b.n_kind64[KIND64_TILE]) k_reset_tiles<<<1, 1, 0, s>>>(io.tile_ctr);
-        if constexpr (MODE == MODE_STEP && KIND == KIND_FIELD) {
-            // more, shorter items: 8 blocks a CU where the tiles had fewer
-            const int most = 8 * device_cus();
-            if (blocks < most) blocks = 2 * blocks < most ? 2 * blocks : most;
-            launch_walk64s<MODE, KIND, COUNT, SPLIT64>(b, blocks, io, s);
-            k_sum_parts<SPLIT64><<<(b.t_cap + BT - 1) / BT, BT, 0, s>>>(b.P, b.st, io);
-        } else {
-            launch_walk64s<MODE, KIND, COUNT, 1>(b, blocks, io, s);
-        }
+        // more, shorter items: 8 blocks a CU where the tiles had fewer
+        const int most = 8 * device_cus();
+        if (blocks < most) blocks = 2 * blocks < most ? 2 * blocks : most;
+        launch_walk64s<MODE, KIND, COUNT, SPLIT64>(b, blocks, io, s);
+        k_sum_parts<SPLIT64><<<(b.t_cap + BT - 1) / BT, BT, 0, s>>>(b.P, b.st, io);
     }
 }
 
@@ -2072,7 +2070,11 @@ void launch_epe(Bufs& b, hipStream_t s)
     io.dip64 = b.dip64;
     k_reset_tiles<<<1, 1, 0, s>>>(&b.g->tile_ctr2);
     const uint32_t nb = (b.n_total + BT - 1) / BT;
-    const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
+    // at least 4 blocks a CU, also where the float32 walk has 2 (450k particles,
+    // theta 0.15: 40 ms with 2, 29 with 4)
+    const uint32_t few = 4u * (uint32_t)device_cus();
+    const uint32_t most = b.walk_blocks > few ? b.walk_blocks : few;
+    const int blocks = (int)(nb < most ? nb : most);
     k_grain_init<MODE_EPE, KIND_EPE><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
     launch_walk64<MODE_EPE, KIND_EPE>(b, blocks, b.n_total, io, s);
     k_epe_partial<<<dim3(EPE_BLOCKS, b.n_inst), BT, 0, s>>>(b.P, b.st, b.phi, b.epe_part);

@@ -1,0 +1,78 @@
+"""Which float64 walk an instance takes: 2 targets a wavefront, or, where the
+opening angle is small for the size, 64 targets shared by four wavefronts.  The
+counters tell the two apart: a range that a target opens is fetched once for
+the targets of a wavefront, so 2 targets fetch at least half as many ranges as
+targets open, and 64 a small part of that, although the walks' sets are the
+same.  At theta = 0 every target meets every particle, and a walk of 2 targets
+takes several times one of 64 from some 100000 particles on.  Where the walks
+are new to a size, the step's field is the point field (as in
+test_gpu_walk_split.py); and the energies of a record step, whose walk has 1 or
+64 targets a wavefront, are those of the potentials at the particles."""
+import numpy as np
+import pytest
+
+from gpu_common import big_case, gpu_ctx, oracle_sim
+from test_gpu_walk_split import _check
+
+from pot_amd import potg as G
+
+pytestmark = pytest.mark.gpu
+
+
+def shares_tiles(ctx):
+    """of a context with one float64 instance, after steps since its counters
+    were reset"""
+    st = ctx.stats()
+    return 4 * st["n_range_loads"] < st["n_open"]
+
+
+@pytest.mark.parametrize("N,theta,dipoles,shared", [
+    (20001, 0.0, 1, False), (120001, 0.0, 1, True), (200001, 0.03, 0, True),
+    (200001, 0.05, 1, True), (200001, 0.12, 1, False), (300001, 0.0, 0, True),
+    (450001, 0.05, 1, True), (450001, 0.11, 0, True), (450001, 0.2, 1, False),
+    (500001, 0.12, 0, True), (500001, 0.14, 1, True), (500001, 0.2, 1, False)])
+def test_kind_by_angle_and_size(N, theta, dipoles, shared):
+    case = dict(big_case(N, seed=31), theta=theta, dipoles=dipoles)
+    ctx = gpu_ctx(case, oracle_sim(case).particles(), q=-30)
+    ctx.step()
+    assert shares_tiles(ctx) == shared, ctx.stats()
+
+
+@pytest.mark.parametrize("N,theta,geometry,dipoles", [(120002, 0.02, 0, 1), (200001, 0.0, 0, 0),
+                                                      (300001, 0.08, 1, 1)])
+def test_shared_tiles_of_smaller_instances(N, theta, geometry, dipoles):
+    case = dict(big_case(N, geometry=geometry, A=2.0 if geometry else 1.0, seed=32), theta=theta,
+                dipoles=dipoles)
+    _check(case, oracle_sim(case).particles())
+
+
+QE, K4PE0 = 1.6021766e-19, 4.0 * np.pi * 8.85419e-12
+
+
+@pytest.mark.parametrize("prec", [G.POTG_FP64, G.POTG_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("N,theta,dipoles", [(60001, 0.01, 1), (60001, 0.2, 1), (250001, 0.09, 0),
+                                             (500001, 0.12, 1), (500001, 0.13, 0)])
+def test_energies_are_the_potentials(prec, N, theta, dipoles):
+    """Particles at rest are not drifted, so a particle's potential is that of a
+    point query at its place but for its own leaf's q / soft.  (At these angles
+    no cell that holds a target is far enough from it to be taken whole.)  Both
+    walks are exact to some roundings of each term: 1e-13 of the terms' sum,
+    which is below that of the leaves' own plus N / R each."""
+    case = dict(big_case(N, seed=33), theta=theta, dipoles=dipoles)
+    parts = oracle_sim(case).particles()
+    for f in ("vx", "vy", "vz"):
+        parts[f] = 0.0
+    ctx = gpu_ctx(case, parts, precision=prec, q=-30)
+    ctx.build_tree()
+    phi = ctx.phi_at(0, np.stack([parts[f] for f in ("x", "y", "z")], 1))
+    ctx = gpu_ctx(case, parts, precision=prec, q=-30)
+    ctx.step(1)
+    epe = ctx.download(0)[1]["epe"]
+    q = np.array([-30.0, 1.0, -1.0])[parts["species"]]
+    own = QE * q / (K4PE0 * float(case["args"]["-s"]))
+    R = float(case["args"]["-r"]) * float(case["args"]["-m"])
+    for s in (G.ION, G.ELECTRON):
+        k = parts["species"] == s
+        want = float((QE * q[k] * (phi[k] - own[k])).sum())
+        mag = float((QE * (np.abs(own[k]) + QE / K4PE0 * 4.0 * N / R)).sum())
+        assert abs(epe[s] - want) <= 1e-13 * mag, (s, epe[s], want, mag)
