@@ -211,21 +211,20 @@ void fill_params(InstParams& p, const potg_config& k)
 //   0.13   3.4/7.9 5.8/10  8.2/13   15/18    25.8/24.1
 //   0.14                                     21.3/21.0  24.7/23.2/27.2
 //   theta  1M             2M              4M       8M       16M
-//   0.14   60/40/43       146/77/80
-//   0.20   21.6/21.1      50/38
-//   0.25   11.0/12.9      24.4/24.0/24.3
-//   0.31                                  27/29
+//   0.14   60/40/43       146/76.5/76.6   /152/143
+//   0.20   21.6/21.1      50/37.1/37.1             /140/131
+//   0.25   11.0/12.9      24.4/26.1/25.0  /44.3/42.4
+//   0.30                                  /29/     /58/54
 //   0.33                                           47.8/47.9
-//   0.38                                                    67/72
-// so the crossing is put at theta = c + 0.05 log2(N / 1M), the parts' gain
-// over a whole tile goes down with the size, and their sums take 96 bytes a
-// particle: up to 32M particles.  By an instance's own values, so that its walk
-// is the same alone and in a batch.
+//   0.38                                                    67/72/65
+// so the crossing is put at theta = c + 0.05 log2(N / 1M), and tiles are shared
+// below 2M particles.  By an instance's own values, so that its walk is the
+// same alone and in a batch.
 int kind64_rule(const InstParams& p)
 {
     if (sqrt(p.theta2) >= (p.dipoles ? 0.201 : 0.171) + 0.05 * log2((double)p.tree_n / 1e6))
         return KIND64_FEW;
-    return p.tree_n < 32000000u ? KIND64_SPLIT : KIND64_TILE;
+    return p.tree_n < 2000000u ? KIND64_SPLIT : KIND64_TILE;
 }
 
 // The same for the potential-energy walk, which has one target a wavefront (no
@@ -563,7 +562,10 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
     rc |= alloc_n(c, &b.t_first, n_inst) | alloc_n(c, &b.t_base, n_inst);
     rc |= alloc_n(c, &b.queue, nt);
     rc |= alloc_n(c, &b.E, 3 * tc) | alloc_n(c, &b.inv, n);
-    if (precision == POTG_FP64 && b.n_kind64[KIND64_SPLIT]) rc |= alloc_n(c, &b.parts, 3 * SPLIT64 * tc);
+    if (precision == POTG_FP64 && b.n_kind64[KIND64_SPLIT]) {
+        b.part_cap = tc < PARTS_MAX ? (uint32_t)tc : PARTS_MAX;
+        rc |= alloc_n(c, &b.parts, 3 * SPLIT64 * (size_t)b.part_cap);
+    }
     b.integrator = configs[0].integrator;
     if (b.integrator != POTG_BORIS) rc |= alloc_n(c, &b.a1, 3 * tc) | alloc_n(c, &b.x0, 3 * tc);
     bool any_bounce = false;

@@ -29,6 +29,9 @@ constexpr uint32_t MOM_GROUP = 32, MOM_ONE = 160;
 // / 2M particles: by level 95 / 105 / 109 / 131 / 277, here 38 / 78 / 95 /
 // 122 / 360
 constexpr uint32_t MOM_MAX = 600000;
+// targets whose shared tiles' partial sums (96 bytes each) are held at a time:
+// those of any one instance that shares its tiles, 200 MB, and a batch's by turns
+constexpr uint32_t PARTS_MAX = 1u << 21;
 inline uint32_t moment_blocks(uint32_t cap) { return (cap + MOM_NODES - 1) / MOM_NODES; }
 // The moment pass' nodes that reach into the next block, by group of blocks,
 // and of these the ones that reach into the next group
@@ -54,7 +57,8 @@ struct Bufs {
     int any_spheroid;  // some instance has the analytic spheroid grain
     int any_bare;      // some instance's tree has no internal nodes
     uint32_t n_kind64[3], n_epe64[3];  // instances by kind64 and kind64_epe
-    double* parts;     // partial sums of the float64 walk's shared tiles
+    double* parts;     // partial sums of the float64 walk's shared tiles, of
+    uint32_t part_cap; // so many targets at a time
     int count;         // step walks keep the interaction counters (potg_set_counting)
     int key_levels;    // digits carried by a sort key
     int key_bits;      // bits of the key that are sorted

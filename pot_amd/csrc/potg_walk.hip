@@ -60,7 +60,8 @@ struct WalkIO {
     // the targets of the instances whose float64 walk is of this kind
     // (InstParams::kind64, kind64_epe), or of all (PICK_ALL)
     int32_t pick;
-    double* parts;     // a split float64 walk's partial sums
+    double* parts;     // a split float64 walk's partial sums, of the targets
+    uint32_t k0, kn;   // from k0 on, kn at most
 };
 constexpr int32_t PICK_ALL = -1;
 
@@ -188,7 +189,8 @@ __device__ inline uint32_t part_share(uint32_t part, uint32_t j)
 // SPLIT: wavefronts that share a tile, each a part of the cells two levels
 // below the root (k_sum_parts adds their sums): with 500k particles a tile a
 // wavefront leaves the device half empty at the end, DIPOLES at theta 0.14
-// 27.2 ms, in four parts 23.2 (1M particles 43.4 and 40.2, 2M 79.6 and 76.7)
+// 27.2 ms, in four parts 23.2 (1M particles 43.4 and 40.2, 2M 76.6 and 76.5, 4M
+// 143 and 152)
 template <int MODE, int KIND, bool DIP, bool COUNT, int SPLIT>
 __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P, Globals* g,
                                                 PState st, const NodeRec64* __restrict__ rec,
@@ -201,6 +203,9 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
     const int wv = threadIdx.x / WAVE;
     const uint32_t lane = __lane_id();
     const uint32_t ntg = (MODE == MODE_STEP) ? *io.n_targets_dev : io.n_pts;
+    // the targets of this launch
+    const uint32_t k0 = SPLIT > 1 ? io.k0 : 0u, left = ntg > k0 ? ntg - k0 : 0u;
+    const uint32_t n_here = SPLIT > 1 && io.kn < left ? io.kn : left;
     unsigned long long tot_cell = 0, tot_leaf = 0, tot_open = 0, tot_pops = 0;
 
     for (;;) {
@@ -208,8 +213,8 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
         if (lane == 0) item = atomicAdd(io.tile_ctr, 1u);
         item = rfl(__shfl(item, 0, WAVE));
         const uint32_t tile = item / SPLIT, part = item % SPLIT;
-        if ((uint64_t)tile * WAVE >= ntg || rfl(step_failed(g) ? 1u : 0u)) break;
-        const uint32_t k = tile * WAVE + lane;
+        if ((uint64_t)tile * WAVE >= n_here || rfl(step_failed(g) ? 1u : 0u)) break;
+        const uint32_t k = k0 + tile * WAVE + lane;
         uint32_t inst, self;
         double tx, ty, tz;
         const bool valid = load_target<MODE, MODE != MODE_POINTS>(P, st, io, k, ntg, inst, self, tx, ty, tz);
@@ -386,7 +391,7 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
         if (valid) {
             const double K = QE / K4PE0;
             if (SPLIT > 1) {
-                double* o = io.parts + 3 * ((size_t)part * ntg + k);
+                double* o = io.parts + 3 * ((size_t)part * io.kn + (k - k0));
                 o[0] = ex;
                 o[1] = ey;
                 o[2] = ez;
@@ -421,15 +426,15 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
 template <int SPLIT>
 __global__ __launch_bounds__(BT) void k_sum_parts(const InstParams* __restrict__ P, PState st, WalkIO io)
 {
-    const uint32_t k = blockIdx.x * BT + threadIdx.x, ntg = *io.n_targets_dev;
-    if (k >= ntg) return;
+    const uint32_t j = blockIdx.x * BT + threadIdx.x, k = io.k0 + j, ntg = *io.n_targets_dev;
+    if (j >= io.kn || k >= ntg) return;
     const uint32_t i = io.targets[k];
     if (i == NONE || !picked(P[st.inst[i]].kind64, io.pick)) return;
     const double K = QE / K4PE0;
     for (int d = 0; d < 3; d++) {
         double e = 0.0;
 #pragma unroll
-        for (int p = 0; p < SPLIT; p++) e += io.parts[3 * ((size_t)p * ntg + k) + d];
+        for (int p = 0; p < SPLIT; p++) e += io.parts[3 * ((size_t)p * io.kn + j) + d];
         io.out[3 * (size_t)k + d] = (io.acc ? io.out[3 * (size_t)k + d] : 0.0) + K * e;
     }
 }
@@ -1972,8 +1977,12 @@ static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream
         // more, shorter items: 8 blocks a CU where the tiles had fewer
         const int most = 8 * device_cus();
         if (blocks < most) blocks = 2 * blocks < most ? 2 * blocks : most;
-        launch_walk64s<MODE, KIND, COUNT, SPLIT64>(b, blocks, io, s);
-        k_sum_parts<SPLIT64><<<(b.t_cap + BT - 1) / BT, BT, 0, s>>>(b.P, b.st, io);
+        io.kn = b.part_cap;
+        for (io.k0 = 0; io.k0 < n; io.k0 += io.kn) {
+            if (io.k0) k_reset_tiles<<<1, 1, 0, s>>>(io.tile_ctr);
+            launch_walk64s<MODE, KIND, COUNT, SPLIT64>(b, blocks, io, s);
+            k_sum_parts<SPLIT64><<<(io.kn + BT - 1) / BT, BT, 0, s>>>(b.P, b.st, io);
+        }
     }
 }
 

@@ -7,11 +7,14 @@ same.  At theta = 0 every target meets every particle, and a walk of 2 targets
 takes several times one of 64 from some 100000 particles on.  Where the walks
 are new to a size, the step's field is the point field (as in
 test_gpu_walk_split.py); and the energies of a record step, whose walk has 1 or
-64 targets a wavefront, are those of the potentials at the particles."""
+64 targets a wavefront, are those of the potentials at the particles.  From 2M
+particles on a tile of 64 has one wavefront.  The shared tiles' partial sums are
+held for 2^21 targets at a time, so that batches of any size find the memory."""
 import numpy as np
 import pytest
+import torch
 
-from gpu_common import big_case, gpu_ctx, oracle_sim
+from gpu_common import big_case, gpu_config, gpu_ctx, oracle_sim
 from test_gpu_walk_split import _check
 
 from pot_amd import potg as G
@@ -76,3 +79,52 @@ def test_energies_are_the_potentials(prec, N, theta, dipoles):
         want = float((QE * q[k] * (phi[k] - own[k])).sum())
         mag = float((QE * (np.abs(own[k]) + QE / K4PE0 * 4.0 * N / R)).sum())
         assert abs(epe[s] - want) <= 1e-13 * mag, (s, epe[s], want, mag)
+
+
+@pytest.mark.parametrize("N,theta", [(2000001, 0.2), (2100001, 0.24)])
+def test_whole_tiles_of_large_instances(N, theta):
+    case = dict(big_case(N, seed=34), theta=theta, dipoles=1)
+    _check(case, oracle_sim(case).particles())
+
+
+def _bytes_of(configs):
+    free0 = torch.cuda.mem_get_info()[0]
+    ctx = G.Context(configs, G.POTG_FP64)
+    used = free0 - torch.cuda.mem_get_info()[0]
+    ctx.close()
+    return used
+
+
+def test_memory_of_shared_tiles_is_bounded():
+    """30M particles in instances that share tiles, against the same with a
+    wide angle: 96 bytes for each of 2^21 targets and allocation granules more."""
+    cases = [dict(big_case(1000001, seed=35), theta=t) for t in (0.1, 0.9)]
+    shared, few = (_bytes_of([gpu_config(c)] * 30) for c in cases)
+    assert 0 <= shared - few <= 96 * 2 ** 21 + 2 ** 25, (shared, few)
+
+
+def test_batch_of_more_targets_than_parts():
+    """Five instances whose targets, stepped all at once (step 42, when the ions
+    are due), fill the parts two and a half times, one of them walked 2 by 2:
+    each ends as it does alone, bit for bit."""
+    case = dict(big_case(1000001, seed=36), theta=0.15)
+    wide = dict(big_case(300001, seed=37), theta=0.9)
+    parts, pw = oracle_sim(case).particles(), oracle_sim(wide).particles()
+    batch = G.Context([gpu_config(case, 7)] * 3 + [gpu_config(wide, 8)] + [gpu_config(case, 7)] * 2,
+                      G.POTG_FP64)
+    one = [G.Context([gpu_config(c, s)], G.POTG_FP64) for c, s in ((case, 7), (wide, 8))]
+    for k in (0, 1, 2, 4, 5):
+        batch.upload(k, parts.view(G.PARTICLE_DT), q=-30, t=41)
+    batch.upload(3, pw.view(G.PARTICLE_DT), q=-30, t=41)
+    one[0].upload(0, parts.view(G.PARTICLE_DT), q=-30, t=41)
+    one[1].upload(0, pw.view(G.PARTICLE_DT), q=-30, t=41)
+    out = batch.step()
+    assert sum(o["n_pushed"] for o in out) > 2.5 * 2 ** 21
+    want = []
+    for c in one:
+        c.step()
+        want.append(c.download(0))
+    for k in range(6):
+        p, g = batch.download(k)
+        pw_, gw = want[k == 3]
+        assert np.array_equal(p.view(np.uint8), pw_.view(np.uint8)) and g == gw, k
