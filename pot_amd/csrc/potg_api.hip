@@ -469,9 +469,10 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
     // - below 1 (under about 32k particles) the tiles would leave most SIMDs
     //   idle: 8 targets per wavefront with 8 children evaluated at once, 2
     //   blocks per CU.
-    // The float64 walk has one shape: 64 targets, 8 blocks per CU from 16
-    // tiles per CU, 4 below.
-    {
+    // The float64 walk's shape is each instance's own (kind64_rule); tiles of 64
+    // targets have 8 blocks per CU from 16 per CU or where wavefronts share
+    // them, 4 below.
+    const auto default_shape = [&]() {
         const uint64_t cus = (uint64_t)device_cus();
         const uint64_t tiles = n_total / 128u;
         const bool large = tiles >= 16u * cus, tiny = tiles < cus;
@@ -480,11 +481,12 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
             b.group = tiny ? 8u : 64u;
             b.variant = tiny ? 0u : 1u;
         } else {
-            b.walk_blocks = (large ? 8u : 4u) * (uint32_t)cus;
+            const bool shared = precision == POTG_FP64 && b.n_kind64[KIND64_SPLIT] != 0;
+            b.walk_blocks = (large || shared ? 8u : 4u) * (uint32_t)cus;
             b.group = 64u;
             b.variant = 0u;
         }
-    }
+    };
 
     c->hp.resize(n_inst);
     uint32_t off = 0, tb = 0;
@@ -501,6 +503,7 @@ int potg_create(const potg_config* configs, uint32_t n_inst, int32_t precision, 
         off += (uint32_t)configs[i].N;
         tb += c->hp[i].tree_n;
     }
+    default_shape();
 
     const size_t n = b.n_total, nt = b.n_tree ? b.n_tree : 1;
     int rc = 0;
@@ -1133,19 +1136,23 @@ int potg_tune(potg_ctx* c, potg_tuning* out)
     // 8, 16, or 64 in either order) x blocks per CU
     const uint32_t shapes[][2] = {{8, 0}, {16, 0}, {64, 0}, {64, 1}};
     const uint32_t bpc[] = {2, 4, 8, 16};
+    // the grid of a float64 walk of 2 targets a wavefront is its size's alone:
+    // one timing, for walk_ms
+    const bool one_grid = b.precision == POTG_FP64 && b.n_kind64[KIND64_FEW] == b.n_inst;
     const uint32_t keep_wb = b.walk_blocks, keep_gr = b.group, keep_var = b.variant;
     double best = 1e30, keep_ms = -1.0;
     uint32_t best_wb = keep_wb, best_gr = keep_gr, best_var = keep_var;
     hipEvent_t e0 = c->ev[0], e1 = c->ev[1];
     for (uint32_t wb : bpc) {
+        if (one_grid && wb != bpc[0]) break;
         for (const auto& sh : shapes) {
             const uint32_t gr = sh[0];
-            // the float64 and group-criterion walks have one shape: only the
-            // grid varies
+            // the float64 walk's shape is its instances' own, and the
+            // group-criterion walk has one: only the grid varies
             if (b.precision != POTG_MIXED && (gr != 64 || sh[1] != 0)) continue;
             b.group = gr;
             b.variant = sh[1];
-            b.walk_blocks = wb * cus;
+            b.walk_blocks = one_grid ? keep_wb : wb * cus;
             float ms_best = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
                 launch_walk_init(b, s);
@@ -1177,10 +1184,10 @@ int potg_tune(potg_ctx* c, potg_tuning* out)
     }
     // the radix sort's tile: the keys, sort and permute of the coming step
     // again under each tile size (the state is sorted already, so the order
-    // stays as it is)
+    // stays as it is); fewer keys than MERGE_MAX are merged, with no tile to choose
     const uint32_t keep_ipt = b.sort_ipt;
     uint32_t best_ipt = keep_ipt;
-    if (!rc) {
+    if (b.n_total >= MERGE_MAX) {
         float sbest = 1e30f, skeep = -1.f;
         for (uint32_t ipt : {8u, 16u}) {
             b.sort_ipt = ipt;

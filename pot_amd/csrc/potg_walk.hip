@@ -1974,9 +1974,6 @@ static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream
     if constexpr (MODE == MODE_STEP) {
         if (!pick(KIND64_SPLIT)) return;
         if (b.n_kind64[KIND64_TILE]) k_reset_tiles<<<1, 1, 0, s>>>(io.tile_ctr);
-        // more, shorter items: 8 blocks a CU where the tiles had fewer
-        const int most = 8 * device_cus();
-        if (blocks < most) blocks = 2 * blocks < most ? 2 * blocks : most;
         io.kn = b.part_cap;
         for (io.k0 = 0; io.k0 < n; io.k0 += io.kn) {
             if (io.k0) k_reset_tiles<<<1, 1, 0, s>>>(io.tile_ctr);
