@@ -10,10 +10,14 @@ namespace potg {
 // it: the first computes its tile's elements and leaves the tile's sum in
 // `part`, the second adds up the sums of the tiles before its own
 // (sum_before: a load or two per thread below a million elements) and scans
-// its tile.  (A launch of its own for the scan of the sums cost 4.5 us.)
+// its tile.  A launch of its own for the scan of the sums costs 4.5 us; adding
+// them up in every block costs the square of their number, which from
+// SCAN_SUMS tiles on is more: tree and targets of 16M / 32M / 64M / 200M particles
+// 3.43 / 7.50 / 16.6 / 91.6 ms without that launch, 3.39 / 7.42 / 17.0 / 82.5 with.
 constexpr int SCAN_BT = 256;               // threads of a scanning block
 constexpr int SCAN_IPT = 4;                // elements per thread
 constexpr int SCAN_TILE = SCAN_BT * SCAN_IPT;
+constexpr uint32_t SCAN_SUMS = 65536;
 inline uint32_t scan_blocks(uint32_t n) { return n ? (n + SCAN_TILE - 1) / SCAN_TILE : 1; }
 
 // inclusive scan across a wavefront
@@ -45,9 +49,15 @@ __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t* sh_w, uint32_t*
     return off + inc - v;
 }
 
+// between a scan's two launches over nb tiles, where that pays: part[b] becomes
+// the sum of part[0..b), and the result is what sum_before takes as `summed`
+int scan_sums(uint32_t* part, uint32_t nb, hipStream_t s);
+
 // the sum of part[0..b), in every thread of the block
-__device__ inline uint32_t sum_before(const uint32_t* __restrict__ part, uint32_t b, uint32_t* sh_w)
+__device__ inline uint32_t sum_before(const uint32_t* __restrict__ part, uint32_t b, int summed,
+                                      uint32_t* sh_w)
 {
+    if (summed) return part[b];
     uint32_t v = 0, total;
     for (uint32_t i = threadIdx.x; i < b; i += SCAN_BT) v += part[i];
     block_excl_scan(v, sh_w, &total);

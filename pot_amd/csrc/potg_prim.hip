@@ -15,6 +15,38 @@ __device__ inline uint32_t lane_id() { return __lane_id(); }
 
 __device__ inline uint64_t lanemask_lt() { return (1ull << lane_id()) - 1ull; }
 
+// exclusive scan of the tile sums, one block: 16 of them a thread in turn, so
+// that 400000 (400M elements) take 25 turns
+__global__ __launch_bounds__(1024) void k_scan_sums(uint32_t* __restrict__ part, uint32_t nb)
+{
+    constexpr int K = 16;
+    __shared__ uint32_t sh_w[1024 / WAVE];
+    uint32_t carry = 0;
+    for (uint32_t b0 = 0; b0 < nb; b0 += 1024u * K) {
+        const uint32_t i0 = b0 + threadIdx.x * K;
+        uint32_t v[K], s = 0;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            v[k] = i0 + k < nb ? part[i0 + k] : 0u;
+            s += v[k];
+        }
+        const uint32_t inc = wave_incl_scan(s);
+        if (lane_id() == WAVE - 1) sh_w[threadIdx.x / WAVE] = inc;
+        __syncthreads();
+        uint32_t off = carry + inc - s;
+        for (uint32_t w = 0; w < 1024 / WAVE; w++) {
+            if (w < threadIdx.x / WAVE) off += sh_w[w];
+            carry += sh_w[w];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (i0 + k < nb) part[i0 + k] = off;
+            off += v[k];
+        }
+    }
+}
+
 // ---- radix sort -------------------------------------------------------
 //
 // 8-bit digits, three launches per pass: the digit counts of every tile of
@@ -237,6 +269,13 @@ __global__ __launch_bounds__(BT) void k_merge(const uint64_t* __restrict__ kin,
 }
 
 }  // namespace
+
+int scan_sums(uint32_t* part, uint32_t nb, hipStream_t s)
+{
+    if (nb < SCAN_SUMS) return 0;
+    k_scan_sums<<<1, 1024, 0, s>>>(part, nb);
+    return 1;
+}
 
 // sized for the smaller tile, which needs more per-tile counts
 size_t radix_temp_words(uint32_t n) { return 256ull * (rs_blocks(n, 8) + 1) + 64; }

@@ -756,14 +756,14 @@ __global__ __launch_bounds__(SCAN_BT) void k_target_flags(const InstParams* __re
 // of 64 with NONE
 __global__ __launch_bounds__(SCAN_BT) void k_target_scan(const uint32_t* __restrict__ flags,
                                                          const uint32_t* __restrict__ part,
-                                                         uint32_t n_tree, int one,
+                                                         int summed, uint32_t n_tree, int one,
                                                          uint32_t* __restrict__ tpos,
                                                          uint32_t* __restrict__ targets, Globals* g)
 {
     __shared__ uint32_t sh[SCAN_TILE];
     __shared__ uint32_t sh_w[SCAN_BT / WAVE];
     const uint32_t t0 = blockIdx.x * SCAN_TILE;
-    const uint32_t off = sum_before(part, blockIdx.x, sh_w);
+    const uint32_t off = sum_before(part, blockIdx.x, summed, sh_w);
     uint32_t f[SCAN_IPT];
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
@@ -1129,7 +1129,9 @@ void launch_targets(Bufs& b, hipStream_t s)
     const uint32_t nb = scan_blocks(b.n_tree);
     const int one = b.n_inst == 1;
     k_target_flags<<<nb, SCAN_BT, 0, s>>>(b.P, b.S, b.st, b.n_tree, b.flags, b.scan_tmp);
-    k_target_scan<<<nb, SCAN_BT, 0, s>>>(b.flags, b.scan_tmp, b.n_tree, one, b.tpos, b.targets, b.g);
+    const int summed = scan_sums(b.scan_tmp, nb, s);
+    k_target_scan<<<nb, SCAN_BT, 0, s>>>(b.flags, b.scan_tmp, summed, b.n_tree, one, b.tpos, b.targets,
+                                         b.g);
     if (one) return;
     k_target_bases<<<1, 1024, 0, s>>>(b.P, b.n_inst, b.n_tree, b.flags, b.tpos, b.t_first,
                                       b.t_base, b.targets, b.g);

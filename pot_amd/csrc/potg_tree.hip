@@ -311,7 +311,7 @@ __global__ __launch_bounds__(SCAN_BT) void k_lcp(const uint64_t* __restrict__ ke
 // the internal nodes, numbered by owner and level (a pre-order)
 __global__ __launch_bounds__(SCAN_BT) void k_nodes(const int32_t* __restrict__ lcp,
                                                    const uint32_t* __restrict__ part,
-                                                   uint32_t n_tree, uint32_t cap,
+                                                   int summed, uint32_t n_tree, uint32_t cap,
                                                    uint32_t* __restrict__ base,
                                                    uint32_t* __restrict__ owner,
                                                    int32_t* __restrict__ level,
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(SCAN_BT) void k_nodes(const int32_t* __restrict__ l
     __shared__ uint32_t sh[SCAN_TILE];
     __shared__ uint32_t sh_w[SCAN_BT / WAVE];
     const uint32_t t0 = blockIdx.x * SCAN_TILE;
-    const uint32_t off = sum_before(part, blockIdx.x, sh_w);
+    const uint32_t off = sum_before(part, blockIdx.x, summed, sh_w);
     if (threadIdx.x == 0) shl[0] = t0 ? lcp[t0 - 1] : -1;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
@@ -498,8 +498,8 @@ __global__ __launch_bounds__(SCAN_BT) void k_ccount(const uint32_t* __restrict__
 // run, the runs in the nodes' order
 __global__ __launch_bounds__(SCAN_BT) void k_wids(const uint32_t* __restrict__ slots,
                                                   const uint32_t* __restrict__ ccount,
-                                                  const uint32_t* __restrict__ part, Globals* g,
-                                                  uint32_t cap, uint32_t n_inst,
+                                                  const uint32_t* __restrict__ part, int summed,
+                                                  Globals* g, uint32_t cap, uint32_t n_inst,
                                                   uint32_t* __restrict__ cfirst,
                                                   uint32_t* __restrict__ wid_int,
                                                   uint32_t* __restrict__ wid_leaf)
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(SCAN_BT) void k_wids(const uint32_t* __restrict__ s
     const uint32_t nint = n_int_of(g, cap), t0 = blockIdx.x * SCAN_TILE;
     if (nint == 0 && t0 == 0 && threadIdx.x == 0) g->n_children = 0;
     if (t0 >= nint) return;
-    const uint32_t off = sum_before(part, blockIdx.x, sh_w);
+    const uint32_t off = sum_before(part, blockIdx.x, summed, sh_w);
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
         const uint32_t j = k * SCAN_BT + threadIdx.x;
@@ -1334,14 +1334,17 @@ void launch_tree(Bufs& b, hipStream_t s)
     const uint32_t cap = b.cap_int;
     k_lcp<<<scan_blocks(n), SCAN_BT, 0, s>>>(b.key, b.st, b.P, n, b.key_levels, b.lcp, b.scan_tmp,
                                              b.g, b.ml);
-    k_nodes<<<scan_blocks(n), SCAN_BT, 0, s>>>(b.lcp, b.scan_tmp, n, cap, b.base, b.owner, b.level,
-                                               b.slots, b.g);
+    int summed = scan_sums(b.scan_tmp, scan_blocks(n), s);
+    k_nodes<<<scan_blocks(n), SCAN_BT, 0, s>>>(b.lcp, b.scan_tmp, summed, n, cap, b.base, b.owner,
+                                               b.level, b.slots, b.g);
     k_link<<<grid(cap > n ? cap : n), BT, 0, s>>>(b.key, b.lcp, b.base, b.owner, b.level, b.st, b.P,
                                                    n, b.key_levels, cap, b.g, b.slots, b.wid_int,
                                                    b.wid_leaf, b.size2);
     k_ccount<<<scan_blocks(cap), SCAN_BT, 0, s>>>(b.slots, b.g, cap, b.ccount, b.scan_tmp);
-    k_wids<<<scan_blocks(cap), SCAN_BT, 0, s>>>(b.slots, b.ccount, b.scan_tmp, b.g, cap, b.n_inst,
-                                                b.cfirst, b.wid_int, b.wid_leaf);
+    // (the sums of tiles past the nodes there are, are never read)
+    summed = scan_sums(b.scan_tmp, scan_blocks(cap), s);
+    k_wids<<<scan_blocks(cap), SCAN_BT, 0, s>>>(b.slots, b.ccount, b.scan_tmp, summed, b.g, cap,
+                                                b.n_inst, b.cfirst, b.wid_int, b.wid_leaf);
     if (!b.ml.group) {
         k_leaf_records<<<grid(n), BT, 0, s>>>(b.st, b.P, b.S, n, b.n_rec, b.wid_leaf, b.rec64, r32,
                                               b.dip64, d32);
