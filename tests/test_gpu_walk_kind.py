@@ -128,3 +128,56 @@ def test_batch_of_more_targets_than_parts():
         p, g = batch.download(k)
         pw_, gw = want[k == 3]
         assert np.array_equal(p.view(np.uint8), pw_.view(np.uint8)) and g == gw, k
+
+
+def test_all_kinds_in_one_context():
+    """A tile for each wavefront, shared tiles and 2 targets a wavefront in one
+    context, whose instances start anywhere in a tile: two steps, the second with
+    its energies (1 or 64 targets a wavefront), end as each does alone, bit for
+    bit."""
+    cases = [dict(big_case(3002, seed=42), theta=0.7), dict(big_case(2000011, seed=43), theta=0.22),
+             dict(big_case(500001, seed=44), theta=0.13, dipoles=1),
+             dict(big_case(20001, seed=45), theta=0.4, dipoles=1),
+             dict(big_case(150001, geometry=1, A=2.0, seed=46), theta=0.04, dipoles=1)]
+    states = [oracle_sim(c).particles().view(G.PARTICLE_DT) for c in cases]
+    batch = G.Context([gpu_config(c, 50 + i) for i, c in enumerate(cases)], G.POTG_FP64)
+    ones = [G.Context([gpu_config(c, 50 + i)], G.POTG_FP64) for i, c in enumerate(cases)]
+    for i, p in enumerate(states):
+        batch.upload(i, p, q=-30)
+        ones[i].upload(0, p, q=-30)
+    for epe in (0, 1):
+        out = batch.step(epe)
+        for i, one in enumerate(ones):
+            assert one.step(epe)[0] == out[i], i
+    for i, one in enumerate(ones):
+        (pb, gb), (po, go) = batch.download(i), one.download(0)
+        assert np.array_equal(pb.view(np.uint8), po.view(np.uint8)) and gb == go, i
+
+
+@pytest.mark.parametrize("n_el", [1, 2, 3, 5, 63, 64, 65, 130, 131])
+@pytest.mark.parametrize("dipoles", [0, 1], ids=["monopole", "dipoles"])
+def test_pairs_of_targets(n_el, dipoles):
+    """Any number of targets, the last of an odd number alone with a wavefront:
+    electrons at rest are moved by dt times the point field (a few roundings,
+    and the sums' order)."""
+    case = dict(big_case(3001, seed=47), dipoles=dipoles)
+    case["args"]["-N"] = str(n_el + 1)
+    R = float(case["args"]["-r"]) * float(case["args"]["-m"])
+    parts = np.zeros(n_el + 1, G.PARTICLE_DT)
+    rng = np.random.default_rng(n_el)
+    for f in ("x", "y", "z"):
+        parts[f] = R
+        parts[f][1:] = R + 0.5 * R * rng.uniform(-1.0, 1.0, n_el)
+    parts["species"][1:] = G.ELECTRON
+    ctx = gpu_ctx(case, parts, q=9)
+    ctx.build_tree()
+    el = np.arange(1, n_el + 1, dtype=np.uint32)
+    E, cnt = ctx.field_at(0, np.stack([parts[f][1:] for f in ("x", "y", "z")], 1), exclude=el, counts=True)
+    ctx.stats_reset()
+    ctx.step()
+    st = ctx.stats()
+    assert [st[k] for k in ("n_cell", "n_leaf", "n_open")] == [int(c) for c in cnt.sum(0, dtype=np.int64)]
+    p = ctx.download(0)[0]
+    v = np.stack([p["v" + f][1:] for f in ("x", "y", "z")], 1)
+    dv = -QE / 9.109383e-31 * float(case["args"]["-d"]) * E
+    assert np.all(np.linalg.norm(v - dv, axis=1) <= 1e-11 * np.linalg.norm(dv, axis=1))
