@@ -142,8 +142,10 @@ typedef struct potg_stats_t {
     uint64_t max_depth;
     uint64_t n_range_loads; /* child ranges fetched by walk wavefronts */
     uint64_t n_child_visits; /* children visited by float32-walk wavefronts (64
-                                targets each): (n_cell + n_leaf) / (64 n_child_visits)
-                                is the fraction of lanes doing an interaction */
+                                targets each; where each of the 64 lanes takes a
+                                child of its own for one target, as in point
+                                queries, the visits of 64 lanes count as one):
+                                (n_cell + n_leaf) / (64 n_child_visits) is the fraction of lanes doing an interaction */
 } potg_stats_t;
 
 /* Launch parameters of the field walk (potg_tune picks them by timing).

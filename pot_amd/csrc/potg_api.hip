@@ -1032,6 +1032,7 @@ int potg_stats(potg_ctx* c, potg_stats_t* out)
         g.n_leaf += q.n[1];
         g.n_open += q.n[2];
         g.n_pops += q.n[3];
+        g.n_visits += q.n[4];
     }
     out->n_cell = g.n_cell;
     out->n_leaf = g.n_leaf;

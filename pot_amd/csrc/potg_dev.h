@@ -127,10 +127,10 @@ struct Globals {
     unsigned long long n_visits; // children visited by float32-walk wavefronts
     uint32_t retire;             // a failed reinjection retires its instance (1) or
                                  // fails the step (0, the default)
-    // the one-target walk's share of n_cell, n_leaf, n_open and n_pops, by
-    // block: tens of thousands of wavefronts adding to one address took
+    // the one-target walk's share of n_cell, n_leaf, n_open, n_pops and n_visits,
+    // by block: tens of thousands of wavefronts adding to one address took
     // longer than the walk (2M targets 17 ms instead of 2.5)
-    struct __align__(64) { unsigned long long n[4]; } lone[128];
+    struct __align__(64) { unsigned long long n[5]; } lone[128];
 };
 constexpr uint32_t LONE_SLOTS = 128;
 

@@ -1104,12 +1104,12 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
     const uint32_t ntg = (MODE == MODE_STEP) ? *io.n_targets_dev : io.n_pts;
     const bool failed = rfl(step_failed(g) ? 1u : 0u) != 0u;
     if (lane < 8u) s_mem[wv][lane] = make_uint2(0u, 0u);
-    __shared__ unsigned long long s_tot[4];
+    __shared__ unsigned long long s_tot[5];
     if constexpr (COUNT && KIND == KIND_FIELD) {
-        if (threadIdx.x < 4u) s_tot[threadIdx.x] = 0ull;
+        if (threadIdx.x < 5u) s_tot[threadIdx.x] = 0ull;
         __syncthreads();
     }
-    unsigned long long tot_cell = 0, tot_leaf = 0, tot_open = 0, tot_pops = 0;
+    unsigned long long tot_cell = 0, tot_leaf = 0, tot_open = 0, tot_pops = 0, tot_vis = 0;
     const uint32_t nblk = (ntg + NW * per_wave - 1) / (NW * per_wave);
     const uint32_t per_xcd = (nblk + XCDS - 1) / XCDS;
 
@@ -1193,6 +1193,7 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
                     const uint32_t w = en.x + (lane_of(m_rng) ? ci * U : 0u);
                     const int base = sp - take;
                     loads += (uint32_t)take;
+                    if (COUNT && !F64) tot_vis++;
                     const uint32_t wr = w / U;
                     Rec r;
                     if constexpr (F64) r = rec[w];
@@ -1365,9 +1366,10 @@ __global__ __launch_bounds__(BT, 8) void k_walk1(const InstParams* __restrict__ 
             atomicAdd(&s_tot[1], tot_leaf);
             atomicAdd(&s_tot[2], tot_open);
             atomicAdd(&s_tot[3], tot_pops);
+            atomicAdd(&s_tot[4], tot_vis);
         }
         __syncthreads();
-        if (threadIdx.x < 4u)
+        if (threadIdx.x < 5u)
             atomicAdd(&g->lone[blockIdx.x % LONE_SLOTS].n[threadIdx.x], s_tot[threadIdx.x]);
     }
 }
