@@ -243,7 +243,7 @@ int potg_phi_at(potg_ctx* ctx, uint32_t inst, const double* xyz, size_t n, doubl
    capture, tight serving loops, harnesses that forbid hipMalloc.  No
    counterpart in the reference.  d_xyz (3 n doubles) and d_phi (n doubles)
    are device memory; the call allocates nothing (its scratch is a fixed
-   array of 0.5 MB per device, held until the process ends), does not
+   array of about 0.5 MB per device, held until the process ends), does not
    synchronise and enqueues on `stream` (a hipStream_t; NULL for the
    context's stream).  n may be at most POTG_NOALLOC_MAX_POINTS, else
    POTG_ERR_ARG.  Calls that overlap on one GPU share the scratch and race.

@@ -247,6 +247,46 @@ int kind64_epe_rule(const InstParams& p)
     return sqrt(p.theta2) >= line ? KIND64_FEW : KIND64_TILE;
 }
 
+// Whether m points walked in the caller's order are near one another: of 256
+// steps from one to the next most are below a quarter of the domain's radius (of
+// random points 1 in 50)
+bool in_order(const InstParams& p, const double* xyz, uint32_t m)
+{
+    uint32_t near = 0;
+    for (uint32_t j = 0; j < 256u; j++) {
+        const double* a = xyz + 3 * (size_t)((uint64_t)j * (m - 1u) / 256u);
+        const double dx = a[3] - a[0], dy = a[4] - a[1], dz = a[5] - a[2];
+        near += dx * dx + dy * dy + dz * dz < 0.0625 * p.R * p.R;
+    }
+    return near > 128u;
+}
+
+// Whether m points of one query share tiles of 64 (k_walk64, k_walk32s) or have a
+// wavefront each (k_walk1).  Sharing takes tens of thousands of points, as a tile
+// is one wavefront's long walk, and a small theta, where neighbours' sets differ
+// little; scattered points' sets are alike only where nearly every node is in
+// them.  ms, a wavefront each / shared, float64, 200k particles (600k for 600k
+// points), DIPOLES, in order | scattered:
+//   points  theta 0    0.04            0.1             0.2        0.3
+//   32k     0.76*      0.55 | 0.48     0.22 | 0.11
+//   65k     1.52       1.14 | 0.95     0.47 | 0.21     0.23 | 0.07
+//   200k    3.40       2.81 | 1.90     1.18 | 0.43     0.59 | 0.14
+//   600k               5.75 | 2.37     2.94 | 0.52     1.32 | 0.22    0.98 | 0.16
+//   4M                                                              1.34
+// (* the times' ratio; float32 within 0.2 of it, and monopoles' lines some 0.02
+// lower; below 50000 particles each alone is as fast at theta 0).  So the lines
+// lie where the ratio is one.  Up to POTG_NOALLOC_MAX_POINTS the points are
+// not looked at: they may be the device's, and potg_phi_at's results are
+// potg_phi_at_noalloc's.
+bool points_share(const InstParams& p, const double* xyz, size_t m)
+{
+    if (m < 49152u || p.tree_n < 50000u) return false;
+    const double theta = sqrt(p.theta2), n = (double)m / 65536.0;
+    if (theta < (p.dipoles ? 0.035 : 0.025) * pow(n, 0.25)) return true;
+    return m > POTG_NOALLOC_MAX_POINTS && theta < (p.dipoles ? 0.045 : 0.02) + 0.065 * log2(n) &&
+           in_order(p, xyz, (uint32_t)m);
+}
+
 // chi_b sampling point of the one worker (measure_chi_b, pot.c:2257-2275)
 void chi_point(InstParams& p)
 {
@@ -914,7 +954,7 @@ static int run_points(potg_ctx* c, uint32_t inst, const double* xyz, const uint3
         if (excl)
             HIPCHK(hipMemcpyAsync(b.q_self, exclude + s0, sizeof(uint32_t) * m, hipMemcpyHostToDevice, c->stream));
         launch_point_targets(b, inst, p.offset, p.N, m, excl, c->stream);
-        launch_points(b, m, kind, c->stream);
+        launch_points(b, m, kind, points_share(p, xyz + 3 * s0, m), c->stream);
         const size_t per = kind == 0 ? 3 : 1;
         HIPCHK(hipMemcpyAsync(out + per * s0, b.q_out, per * sizeof(double) * m, hipMemcpyDeviceToHost, c->stream));
         if (counts && kind == 0)
@@ -994,7 +1034,7 @@ int potg_phi_at_noalloc(potg_ctx* c, uint32_t inst, const double* d_xyz, size_t 
     if (!c->b.noalloc) return set_err("potg_phi_at_noalloc: no scratch on this device"), POTG_ERR_HIP;
     if (n == 0) return POTG_OK;
     launch_phi_noalloc(c->b, c->b.noalloc, inst, d_xyz, (uint32_t)n, d_phi,
-                       stream ? (hipStream_t)stream : c->stream);
+                       points_share(c->hp[inst], nullptr, n), stream ? (hipStream_t)stream : c->stream);
     HIPCHK(hipGetLastError());
     return POTG_OK;
 }

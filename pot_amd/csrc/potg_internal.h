@@ -157,8 +157,9 @@ void launch_build_inverse(Bufs& b, hipStream_t s);
 void launch_init_slots(Bufs& b, hipStream_t s);
 // permute the state back to reference layout (before an upload)
 void launch_unsort(Bufs& b, hipStream_t s);
-// point queries: n points of q_pts with q_inst/q_self; kind 0 field, 1 potential
-void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s);
+// point queries: n points of q_pts with q_inst/q_self; kind 0 field, 1 potential;
+// share: 64 of them a wavefront, in their order, else each alone
+void launch_points(Bufs& b, uint32_t n, int kind, bool share, hipStream_t s);
 // q_inst of n points, and q_self: from the reference indexes that it holds (of
 // N particles from `offset`; larger ones are none), or none without `indexes`
 void launch_point_targets(Bufs& b, uint32_t inst, uint32_t offset, uint32_t N, uint32_t n,
@@ -169,6 +170,6 @@ void launch_direct_sum(Bufs& b, uint32_t inst, uint32_t n_src, uint32_t n, hipSt
 // point-potential walk over the caller's device arrays using it
 int noalloc_scratch(uint32_t** out);
 void launch_phi_noalloc(Bufs& b, uint32_t* scr, uint32_t inst, const double* pts, uint32_t n,
-                        double* out, hipStream_t s);
+                        double* out, bool share, hipStream_t s);
 
 }  // namespace potg

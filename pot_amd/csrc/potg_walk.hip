@@ -402,6 +402,11 @@ __global__ __launch_bounds__(BT) void k_walk64(const InstParams* __restrict__ P,
             } else {
                 io.out[k] = (io.acc ? io.out[k] : 0.0) + K * ex;
             }
+            if (COUNT && MODE == MODE_POINTS) {
+                io.counts[3 * k] = ncell;
+                io.counts[3 * k + 1] = nleaf;
+                io.counts[3 * k + 2] = nopen;
+            }
         }
         tot_cell += ncell;
         tot_leaf += nleaf;
@@ -1912,12 +1917,13 @@ static void launch_walk1(Bufs& b, uint32_t n, const WalkIO& io, hipStream_t s)
 // float32 field walk of the chosen shape: the group criterion
 // (k_walk32grp); groups of 8 or 16 targets (k_walkg); 64 targets sweeping
 // whole ranges (k_walk32s: group 64, variant 1) or visiting a range's cells
-// until some open one (k_walk32).  Point queries take k_walk1 unless groups of
-// 16 or k_walk32 were set.  Instantiated with dipole support only for contexts
+// until some open one (k_walk32).  Point queries take k_walk1, or k_walk32s where
+// points `share` (points_share), unless groups of 16 or k_walk32 were set.
+// Instantiated with dipole support only for contexts
 // holding DIPOLES instances, and with interaction counting (COUNT) for point
 // queries and for step walks while the context counts.
 template <int MODE, bool COUNT>
-static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
+static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s, bool share)
 {
     const bool dip = b.dip32 != nullptr;
 #define POTG_W32(KERNEL) KERNEL<<<blocks, BT, 0, s>>>(b.P, b.g, b.st, b.rec32, io)
@@ -1925,10 +1931,10 @@ static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
         if (dip) POTG_W32((k_walk32grp<MODE, true, COUNT>));
         else POTG_W32((k_walk32grp<MODE, false, COUNT>));
     } else if (b.group == 8 || (b.group == 64 && b.variant == 1)) {
-        if constexpr (MODE == MODE_POINTS) {
-            // in the caller's order, as often as not scattered
-            launch_walk1<1, false, MODE, KIND_FIELD, COUNT>(b, io.n_pts, io, s);
-        } else if (b.group == 8) {
+        if (MODE == MODE_POINTS && !share) {
+            if constexpr (MODE == MODE_POINTS)
+                launch_walk1<1, false, MODE, KIND_FIELD, COUNT>(b, io.n_pts, io, s);
+        } else if (MODE == MODE_STEP && b.group == 8) {
             if (dip) POTG_W32((k_walkg<8, MODE, true, COUNT>));
             else POTG_W32((k_walkg<8, MODE, false, COUNT>));
         } else {
@@ -1946,10 +1952,10 @@ static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
 }
 
 template <int MODE>
-static void launch_walk32(Bufs& b, int blocks, const WalkIO& io, hipStream_t s)
+static void launch_walk32(Bufs& b, int blocks, const WalkIO& io, hipStream_t s, bool share = false)
 {
-    if (MODE == MODE_POINTS || b.count) launch_walk32c<MODE, true>(b, blocks, io, s);
-    else launch_walk32c<MODE, false>(b, blocks, io, s);
+    if (MODE == MODE_POINTS || b.count) launch_walk32c<MODE, true>(b, blocks, io, s, share);
+    else launch_walk32c<MODE, false>(b, blocks, io, s, share);
 }
 
 template <int MODE, int KIND, bool COUNT, int SPLIT>
@@ -2001,7 +2007,30 @@ void launch_walk(Bufs& b, hipStream_t s)
         launch_walk64<MODE_STEP, KIND_FIELD>(b, (int)b.walk_blocks, b.t_cap, io, s);
 }
 
-void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s)
+// blocks of a float64 walk of n targets, 64 a wavefront, that is no step walk: at
+// least 4 a CU, also where the float32 walk has 2 (energies of 450k particles,
+// theta 0.15: 40 ms with 2, 29 with 4)
+static int tile_blocks(const Bufs& b, uint32_t n)
+{
+    const uint32_t nb = n ? (n + BT - 1) / BT : 1, few = 4u * (uint32_t)device_cus();
+    const uint32_t most = b.walk_blocks > few ? b.walk_blocks : few;
+    return (int)(nb < most ? nb : most);
+}
+
+// float64 walk of points, alone or 64 a wavefront
+template <int KIND>
+static void launch_points64(Bufs& b, uint32_t n, const WalkIO& io, bool share, hipStream_t s)
+{
+    constexpr bool COUNT = KIND == KIND_FIELD;
+    if (!share) {
+        launch_walk1<1, true, MODE_POINTS, KIND, COUNT>(b, n, io, s);
+        return;
+    }
+    k_reset_tiles<<<1, 1, 0, s>>>(io.tile_ctr);
+    launch_walk64s<MODE_POINTS, KIND, COUNT, 1>(b, tile_blocks(b, n), io, s);
+}
+
+void launch_points(Bufs& b, uint32_t n, int kind, bool share, hipStream_t s)
 {
     WalkIO io{};
     io.pts = b.q_pts;
@@ -2018,16 +2047,16 @@ void launch_points(Bufs& b, uint32_t n, int kind, hipStream_t s)
     const uint32_t nb = (n + BT - 1) / BT ? (n + BT - 1) / BT : 1;
     if (kind == 1) {
         if (io.acc) k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-        launch_walk1<1, true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
+        launch_points64<KIND_PHI>(b, n, io, share, s);
         return;
     }
     if (io.acc) k_grain_init<MODE_POINTS, KIND_FIELD><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
     if (b.precision) {
         k_reset_tiles<<<1, 1, 0, s>>>(&b.g->tile_ctr2);
         const int blocks = (int)nb < (int)b.walk_blocks ? (int)nb : (int)b.walk_blocks;
-        launch_walk32<MODE_POINTS>(b, blocks, io, s);
+        launch_walk32<MODE_POINTS>(b, blocks, io, s, share);
     } else {
-        launch_walk1<1, true, MODE_POINTS, KIND_FIELD, true>(b, n, io, s);
+        launch_points64<KIND_FIELD>(b, n, io, share, s);
     }
 }
 
@@ -2078,13 +2107,8 @@ void launch_epe(Bufs& b, hipStream_t s)
     io.dip64 = b.dip64;
     k_reset_tiles<<<1, 1, 0, s>>>(&b.g->tile_ctr2);
     const uint32_t nb = (b.n_total + BT - 1) / BT;
-    // at least 4 blocks a CU, also where the float32 walk has 2 (450k particles,
-    // theta 0.15: 40 ms with 2, 29 with 4)
-    const uint32_t few = 4u * (uint32_t)device_cus();
-    const uint32_t most = b.walk_blocks > few ? b.walk_blocks : few;
-    const int blocks = (int)(nb < most ? nb : most);
     k_grain_init<MODE_EPE, KIND_EPE><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-    launch_walk64<MODE_EPE, KIND_EPE>(b, blocks, b.n_total, io, s);
+    launch_walk64<MODE_EPE, KIND_EPE>(b, tile_blocks(b, b.n_total), b.n_total, io, s);
     k_epe_partial<<<dim3(EPE_BLOCKS, b.n_inst), BT, 0, s>>>(b.P, b.st, b.phi, b.epe_part);
 }
 
@@ -2194,13 +2218,15 @@ void launch_chi_b(Bufs& b, hipStream_t s)
 // ---- point potentials with no allocation (potg_phi_at_noalloc) -----------
 //
 // The walk of a point query reads, besides the caller's points and result
-// array, an instance and excluded-slot entry per point.  For callers that
-// cannot allocate, that scratch is this array: the points' instances, then
-// their excluded slots (all NONE: a potential counts every leaf).  Each device holds one
+// array, a tile counter and an instance and excluded-slot entry per point.
+// For callers that cannot allocate, that scratch is this array: the tile counter,
+// then the points' instances, then their excluded slots (all NONE: a potential
+// counts every leaf).  Each device holds one
 // copy until the process ends; the host reaches it only through the address
 // hipGetSymbolAddress gives on that device.  Calls that overlap on one device
 // share it and race.
-constexpr uint32_t NOALLOC_WORDS = 2 * POTG_NOALLOC_MAX_POINTS;
+constexpr uint32_t NOALLOC_HEAD = 64;  // words before the per-point arrays
+constexpr uint32_t NOALLOC_WORDS = NOALLOC_HEAD + 2 * POTG_NOALLOC_MAX_POINTS;
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
 
 namespace {
@@ -2209,8 +2235,8 @@ __global__ void k_noalloc_prep(uint32_t* __restrict__ scr, uint32_t inst, uint32
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) {
-        scr[k] = inst;
-        scr[POTG_NOALLOC_MAX_POINTS + k] = NONE;
+        scr[NOALLOC_HEAD + k] = inst;
+        scr[NOALLOC_HEAD + POTG_NOALLOC_MAX_POINTS + k] = NONE;
     }
 }
 
@@ -2235,12 +2261,13 @@ int noalloc_scratch(uint32_t** out)
 }
 
 void launch_phi_noalloc(Bufs& b, uint32_t* scr, uint32_t inst, const double* pts, uint32_t n,
-                        double* out, hipStream_t s)
+                        double* out, bool share, hipStream_t s)
 {
     WalkIO io{};
     io.pts = pts;
-    io.pt_inst = scr;
-    io.pt_self = scr + POTG_NOALLOC_MAX_POINTS;
+    io.pt_inst = scr + NOALLOC_HEAD;
+    io.pt_self = scr + NOALLOC_HEAD + POTG_NOALLOC_MAX_POINTS;
+    io.tile_ctr = scr;
     io.n_pts = n;
     io.out = out;
     io.acc = b.any_spheroid;
@@ -2249,7 +2276,7 @@ void launch_phi_noalloc(Bufs& b, uint32_t* scr, uint32_t inst, const double* pts
     const uint32_t nb = (n + BT - 1) / BT ? (n + BT - 1) / BT : 1;
     k_noalloc_prep<<<nb, BT, 0, s>>>(scr, inst, n);
     if (io.acc) k_grain_init<MODE_POINTS, KIND_PHI><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-    launch_walk1<1, true, MODE_POINTS, KIND_PHI, false>(b, n, io, s);
+    launch_points64<KIND_PHI>(b, n, io, share, s);
 }
 
 }  // namespace potg
