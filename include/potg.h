@@ -157,7 +157,8 @@ typedef struct potg_stats_t {
    per CU; the float64 walk takes 8 blocks per CU from 16 tiles per CU, or
    where wavefronts share tiles (64 targets and below 2M particles), 4
    otherwise.  They concern step walks (point queries follow a group of 16 or
-   variant 0 only) and, of the float64 ones, those of instances with 64
+   variant 0, and walk_blocks where they share wavefronts, as many points at
+   small opening angles do) and, of the float64 ones, those of instances with 64
    targets per wavefront: an instance whose opening angle is large for its
    size (DIPOLES: 0.15 at 0.5M particles, 0.2 at 1M, 0.25 at 2M) is walked 2
    by 2. */

@@ -5,7 +5,8 @@
 Everything is compiled in-tree into pot_amd/_build/ with hipcc for gfx950
 only.  Flags:
   -ffp-contract=off   no fused multiply-add unless written: the float64
-                      tree build and walk repeat the reference's roundings
+                      tree build and the walks' opening tests repeat the
+                      reference's roundings
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       no packed float32 instructions
   -munsafe-fp-atomics hardware float64 atomic add for the momentum tally

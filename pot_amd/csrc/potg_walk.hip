@@ -1,13 +1,15 @@
 // potg_walk.hip -- Barnes-Hut field and potential walks on gfx950.
 //
-// One wavefront walks the tree for 64 targets that are neighbours in the
-// sort order.  The walk keeps the reference's per-particle opening test
-// (field_particle_feels_at, pot.c:1718-1806): the wave shares one
-// depth-first traversal whose stack entries carry a 64-bit lane mask; at a
-// cell every lane in the mask applies its own MAC, lanes that accept it add
-// the monopole, and lanes that reject it pass the children on with their
-// mask.  Each lane therefore meets exactly the nodes, in exactly the order,
-// that the reference visits for that particle.
+// Every walk keeps the reference's per-particle opening test
+// (field_particle_feels_at, pot.c:1718-1806), so that each target meets exactly
+// the nodes that the reference visits for that particle; the order of a
+// target's sum differs from walk to walk.  Either a wavefront walks for 64
+// targets that are neighbours in the sort order (k_walk64, k_walk32, k_walk32s):
+// it shares one depth-first traversal whose stack entries carry a 64-bit lane
+// mask; at a cell every lane in the mask applies its own MAC, lanes that accept
+// it add it, and lanes that reject it pass the children on with their mask.  Or
+// it walks for few (k_walk1: 1 or 2; k_walkg: 8 or 16) and its lanes hold
+// different nodes.  (k_walk32grp's criterion is its own.)
 //
 // Memory: the children of a node are contiguous records, so a stack entry
 // is a child range.  A range is fetched with one vector load (lane j holds
@@ -16,8 +18,11 @@
 // interrupted by a descent are pushed back (remaining siblings, same mask)
 // on an LDS stack.
 //
-// FP64: every operation repeats the reference's float64 expressions, with
-// float64 instead of x87 accumulation.  MIXED: coordinates relative to the
+// FP64: the opening test is the reference's float64 expression, in its
+// operations; the interactions are float64 with 1 / r from the hardware's
+// reciprocal square root, refined, and float64 instead of x87 accumulation.
+// chi_b's walk (k_chi_b) repeats the reference's expressions and order.
+// MIXED: coordinates relative to the
 // domain centre in units of R, float32 arithmetic with a hardware reciprocal
 // square root, Kahan-compensated per-particle sums, result scaled back in
 // float64.
@@ -1002,9 +1007,10 @@ __global__ __launch_bounds__(BT) void k_walk32s(const InstParams* __restrict__ P
 
 // ---- 1 or 2 targets per wavefront, 64 nodes at once -------------------------
 //
-// Point queries of both precisions, the potential-energy walk and, where few
-// targets a wavefront are the faster shape (KIND64_FEW), the float64 step walk.
-// (The float32 step walks keep k_walkg's and k_walk32s's order of summation.)
+// Point queries of both precisions and, where few targets a wavefront are the
+// faster shape (KIND64_FEW), the potential-energy walk and the float64 step walk.
+// (Queries of many points at small theta share tiles: points_share.  The float32
+// step walks are k_walkg's and k_walk32s's.)
 //
 // The 64 lanes of a wavefront hold 64 nodes: up to 8 child ranges are taken
 // off an LDS stack at once, lane = 8 range + child, the nodes are tested
