@@ -1937,15 +1937,18 @@ static void launch_walk32c(Bufs& b, int blocks, const WalkIO& io, hipStream_t s,
         if (dip) POTG_W32((k_walk32grp<MODE, true, COUNT>));
         else POTG_W32((k_walk32grp<MODE, false, COUNT>));
     } else if (b.group == 8 || (b.group == 64 && b.variant == 1)) {
-        if (MODE == MODE_POINTS && !share) {
-            if constexpr (MODE == MODE_POINTS)
-                launch_walk1<1, false, MODE, KIND_FIELD, COUNT>(b, io.n_pts, io, s);
-        } else if (MODE == MODE_STEP && b.group == 8) {
+        const auto sweep = [&]() {
+            if (dip) POTG_W32((k_walk32s<MODE, true, COUNT>));
+            else POTG_W32((k_walk32s<MODE, false, COUNT>));
+        };
+        if constexpr (MODE == MODE_POINTS) {
+            if (share) sweep();
+            else launch_walk1<1, false, MODE, KIND_FIELD, COUNT>(b, io.n_pts, io, s);
+        } else if (b.group == 8) {
             if (dip) POTG_W32((k_walkg<8, MODE, true, COUNT>));
             else POTG_W32((k_walkg<8, MODE, false, COUNT>));
         } else {
-            if (dip) POTG_W32((k_walk32s<MODE, true, COUNT>));
-            else POTG_W32((k_walk32s<MODE, false, COUNT>));
+            sweep();
         }
     } else if (b.group == 16) {
         if (dip) POTG_W32((k_walkg<16, MODE, true, COUNT>));
@@ -1997,20 +2000,14 @@ static void launch_walk64p(Bufs& b, int blocks, uint32_t n, WalkIO io, hipStream
     }
 }
 
-template <int MODE, int KIND>
-static void launch_walk64(Bufs& b, int blocks, uint32_t n, const WalkIO& io, hipStream_t s)
-{
-    if (b.count) launch_walk64p<MODE, KIND, true>(b, blocks, n, io, s);
-    else launch_walk64p<MODE, KIND, false>(b, blocks, n, io, s);
-}
-
 void launch_walk(Bufs& b, hipStream_t s)
 {
     WalkIO io = step_io(b);
     if (b.precision)
         launch_walk32<MODE_STEP>(b, (int)b.walk_blocks, io, s);
     else
-        launch_walk64<MODE_STEP, KIND_FIELD>(b, (int)b.walk_blocks, b.t_cap, io, s);
+        (b.count ? launch_walk64p<MODE_STEP, KIND_FIELD, true>
+                 : launch_walk64p<MODE_STEP, KIND_FIELD, false>)(b, (int)b.walk_blocks, b.t_cap, io, s);
 }
 
 // blocks of a float64 walk of n targets, 64 a wavefront, that is no step walk: at
@@ -2114,7 +2111,8 @@ void launch_epe(Bufs& b, hipStream_t s)
     k_reset_tiles<<<1, 1, 0, s>>>(&b.g->tile_ctr2);
     const uint32_t nb = (b.n_total + BT - 1) / BT;
     k_grain_init<MODE_EPE, KIND_EPE><<<nb, BT, 0, s>>>(b.P, b.S, b.st, io);
-    launch_walk64<MODE_EPE, KIND_EPE>(b, tile_blocks(b, b.n_total), b.n_total, io, s);
+    // (not among the interactions that are counted)
+    launch_walk64p<MODE_EPE, KIND_EPE, false>(b, tile_blocks(b, b.n_total), b.n_total, io, s);
     k_epe_partial<<<dim3(EPE_BLOCKS, b.n_inst), BT, 0, s>>>(b.P, b.st, b.phi, b.epe_part);
 }
 
